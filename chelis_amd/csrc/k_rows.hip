@@ -47,16 +47,19 @@ struct VecT<double, 2> {
 
 // Streaming rows are read once and written once: NT selects the
 // nontemporal (streaming) cache policy for them; vectors shared by every row
-// (layer norm's gamma and beta) use the default policy.
-template <bool NT, typename Q>
-__device__ inline Q vload(const Q *p) {
-    if constexpr (NT) return __builtin_nontemporal_load(p);
-    else return *p;
+// (layer norm's gamma and beta) use the default policy. The access is
+// aligned to the element only: a 16-byte global access needs no more on
+// gfx950, so rows of any length and start move as vectors.
+template <bool NT, typename T, int V>
+__device__ inline typename VecT<T, V>::type vload(const T *p) {
+    typedef T Q __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+    if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const Q *>(p));
+    else return *reinterpret_cast<const Q *>(p);
 }
-template <bool NT, typename Q>
-__device__ inline void vstore(Q v, Q *p) {
-    if constexpr (NT) __builtin_nontemporal_store(v, p);
-    else *p = v;
+template <typename T, int V>
+__device__ inline void vstore(typename VecT<T, V>::type v, T *p) {
+    typedef T Q __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+    __builtin_nontemporal_store(v, reinterpret_cast<Q *>(p));
 }
 
 template <typename T>
@@ -137,64 +140,145 @@ struct SlowSet<NE, true> {
 template <int NE>
 struct SlowSet<NE, false> {
     static_assert(NE <= 64, "one bit per element");
-    uint64_t bits = 0;
-    __device__ void set(int k, bool slow) { bits |= (uint64_t)slow << k; }
-    __device__ bool any() const { return __any(bits != 0); }
-    __device__ bool has(int k, int) const { return (bits >> k) & 1u; }
+    uint32_t bits[2] = {0, 0};
+    __device__ void set(int k, bool slow) { bits[k >> 5] |= (uint32_t)slow << (k & 31); }
+    // the lane's next flagged element, or -1, taken out of the set
+    __device__ int take() {
+        const int h = bits[0] ? 0 : 1;
+        const uint32_t b = bits[h];
+        bits[h] = b & (b - 1);
+        return b ? 32 * h + __builtin_ctz(b) : -1;
+    }
+    __device__ bool any() const { return __any((bits[0] | bits[1]) != 0); }
+    __device__ bool has(int k, int) const { return (bits[k >> 5] >> (k & 31)) & 1u; }
 };
 
 // The rare correctly rounded fallback stays out of line: inlined 16 times it
 // would dominate the kernel's code.
 __device__ __noinline__ float expf_slow(float x) { return expf_cr_dd(x); }
 
-// Per-row geometry: which row this wave group owns and where it starts.
-template <int W, int R>
+// Per-row geometry: which row this wave group owns and where it starts. A
+// row has W waves of 64 lanes, or (W = 1) L = 16 lanes of a wave that holds
+// four rows. Lanes of a short row past the last one repeat it (every lane of
+// the wave takes part in its lane exchanges) and do not store.
+template <int W, int R, int L>
 struct RowCoord {
+    static_assert(L == 64 || (L == 16 && W == 1), "whole waves, or a quarter of one");
     int lane, wave_in_row, row_in_block, tid_in_row;
     int64_t row;
-    __device__ RowCoord() {
+    bool live;
+    __device__ explicit RowCoord(int64_t rows) {
         const int tid = threadIdx.x;
         lane = tid & 63;
         const int wave = tid >> 6;
         wave_in_row = wave % W;
         row_in_block = wave / W;
-        tid_in_row = wave_in_row * 64 + lane;
+        tid_in_row = L == 64 ? wave_in_row * 64 + lane : lane % L;
         row = (int64_t)blockIdx.x * R + row_in_block;
+        if (L < 64) row = row * (64 / L) + lane / L;
+        live = row < rows;
+        if (L < 64 && !live) row = rows - 1;
     }
 };
 
-template <typename T, int V, int S, int W, bool NT = true>
-__device__ inline void load_row(const T *__restrict__ p, int64_t n, bool vec_ok, int tid_in_row, T pad,
-                                T (&v)[S][V]) {
-    constexpr int SEG = 64 * W * V;
+// Canonical tree sum and plain maximum of one value per lane over the L
+// lanes of a row; every lane gets the result.
+template <int L, typename T>
+__device__ inline T lanes_tree_sum(T x) {
+    if constexpr (L == 64) return wave_tree_sum(x);
+    x = x + dpp_perm<kDppXor1>(x);
+    x = x + dpp_perm<kDppXor2>(x);
+    x = x + dpp_perm<kDppHalfMirror>(x);
+    return x + dpp_perm<kDppMirror>(x);
+}
+template <int L, typename T>
+__device__ inline T lanes_vmax(T x) {
+    if constexpr (L == 64) return wave_vmax(x);
+    x = vmax(x, dpp_perm<kDppXor1>(x));
+    x = vmax(x, dpp_perm<kDppXor2>(x));
+    x = vmax(x, dpp_perm<kDppHalfMirror>(x));
+    return vmax(x, dpp_perm<kDppMirror>(x));
+}
+
+// A row's n elements, padded past n, in two halves: issue() sends the loads,
+// take() waits for them, so a kernel that reads several rows has all of them
+// in flight before it waits for the first. Neither has a branch around a
+// load (a branch there made the compiler wait for one load before the next:
+// layer norm of [20000, 1000] 34.3 against 31.6 us): a lane past the end
+// reads the row's last V elements again. RAGGED serves row lengths that are
+// no multiple of V; there the lane that straddles the end moves those down
+// to its own place. Without PAD an element past n may hold anything.
+template <typename T, int V, int S, int W, int L, bool RAGGED, bool NT = true, bool PAD = true>
+struct RowLoad {
+    static constexpr int SEG = L * W * V;
+    using Q = typename VecT<T, V>::type;
+    const T *p;
+    int n, tid;
+    Q q[S];
+    __device__ RowLoad(const T *row, int count, int tid_in_row) : p(row), n(count), tid(tid_in_row) {}
+    __device__ void issue() {
+        if (RAGGED && n < V) return;
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const int base = s * SEG + tid * V;
+            q[s] = vload<NT, T, V>(p + (base < n - V ? base : n - V));
+        }
+    }
+    __device__ void take(T pad, T (&v)[S][V]) {
+        if (RAGGED && n < V) {
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+#pragma unroll
+                for (int i = 0; i < V; ++i) {
+                    const int j = s * SEG + tid * V + i;
+                    v[s][i] = j < n ? p[j] : pad;
+                }
+            return;
+        }
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const int base = s * SEG + tid * V;
+            if constexpr (!RAGGED) {
+#pragma unroll
+                for (int i = 0; i < V; ++i) v[s][i] = !PAD || base < n ? q[s][i] : pad;
+            } else {
+                // d elements of the lane's vector lie past the end
+                const int d = base > n - V ? base - (n - V) : 0;
+#pragma unroll
+                for (int i = 0; i < V; ++i) {
+                    v[s][i] = pad;
+#pragma unroll
+                    for (int u = V - 1; u >= i; --u) v[s][i] = i + d == u ? q[s][u] : v[s][i];
+                }
+            }
+        }
+    }
+};
+
+// DENSE: the row is exactly the register capacity.
+template <typename T, int V, int S, int W, int L>
+__device__ inline void load_dense(const T *__restrict__ p, int tid_in_row, T (&v)[S][V]) {
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-        const int64_t base = (int64_t)s * SEG + (int64_t)tid_in_row * V;
-        if (vec_ok && base + V <= n) {
-            typename VecT<T, V>::type q = vload<NT>(reinterpret_cast<const typename VecT<T, V>::type *>(p + base));
-            const T *qe = reinterpret_cast<const T *>(&q);
+        const typename VecT<T, V>::type q =
+            vload<true, T, V>(p + s * L * W * V + tid_in_row * V);
 #pragma unroll
-            for (int i = 0; i < V; ++i) v[s][i] = qe[i];
-        } else {
-#pragma unroll
-            for (int i = 0; i < V; ++i) v[s][i] = (base + i < n) ? p[base + i] : pad;
-        }
+        for (int i = 0; i < V; ++i) v[s][i] = q[i];
     }
 }
 
-template <typename T, int V, int S, int W>
-__device__ inline void store_row(T *__restrict__ p, int64_t n, bool vec_ok, int tid_in_row, const T (&v)[S][V]) {
-    constexpr int SEG = 64 * W * V;
+template <typename T, int V, int S, int W, int L, bool RAGGED>
+__device__ inline void store_row(T *__restrict__ p, int n, int tid_in_row, const T (&v)[S][V]) {
+    constexpr int SEG = L * W * V;
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-        const int64_t base = (int64_t)s * SEG + (int64_t)tid_in_row * V;
-        if (vec_ok && base + V <= n) {
+        const int base = s * SEG + tid_in_row * V;
+        if (base + V <= n) {
             typename VecT<T, V>::type q;
-            T *qe = reinterpret_cast<T *>(&q);
 #pragma unroll
-            for (int i = 0; i < V; ++i) qe[i] = v[s][i];
-            vstore<true>(q, reinterpret_cast<typename VecT<T, V>::type *>(p + base));
-        } else {
+            for (int i = 0; i < V; ++i) q[i] = v[s][i];
+            vstore<T, V>(q, p + base);
+        } else if constexpr (RAGGED) {
 #pragma unroll
             for (int i = 0; i < V; ++i)
                 if (base + i < n) p[base + i] = v[s][i];
@@ -202,22 +286,44 @@ __device__ inline void store_row(T *__restrict__ p, int64_t n, bool vec_ok, int 
     }
 }
 
-// Canonical tree over the padded row; every thread of the row gets the total.
-template <typename T, int V, int S, int W, int R>
-__device__ inline T row_tree_sum(const T (&v)[S][V], T *lds, const RowCoord<W, R> &c) {
+// Canonical tree over the padded row of leaves leaf(s, i); every thread of
+// the row gets the total.
+template <typename T, int V, int S, int W, int R, int L, class F>
+__device__ inline T row_tree_sum(F leaf, T *lds, const RowCoord<W, R, L> &c) {
     T seg[S];
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         T a[V];
 #pragma unroll
-        for (int i = 0; i < V; ++i) a[i] = v[s][i];
+        for (int i = 0; i < V; ++i) a[i] = leaf(s, i);
 #pragma unroll
         for (int w = V; w > 1; w >>= 1)
 #pragma unroll
             for (int i = 0; i < w / 2; ++i) a[i] = a[2 * i] + a[2 * i + 1];
-        seg[s] = wave_tree_sum(a[0]);
+        seg[s] = lanes_tree_sum<L>(a[0]);
     }
-    if constexpr (W > 1) {
+    if constexpr (S * W >= 32 && W > 1) {
+        // the (segment, wave) totals in order are the leaves of the row's top
+        // subtree: each lane joins its run of them and the wave joins the
+        // lanes (-0 past the end). Each thread reading all S * W totals held
+        // too many registers for rows of sixteen waves.
+        constexpr int N = S * W, P = N > 64 ? N / 64 : 1;
+        T *top = lds + c.row_in_block * N;
+        if (c.lane == 0)
+#pragma unroll
+            for (int s = 0; s < S; ++s) top[s * W + c.wave_in_row] = seg[s];
+        __syncthreads();
+        T a[P];
+#pragma unroll
+        for (int i = 0; i < P; ++i) a[i] = c.lane * P + i < N ? top[c.lane * P + i] : T(-0.0);
+#pragma unroll
+        for (int w = P; w > 1; w >>= 1)
+#pragma unroll
+            for (int i = 0; i < w / 2; ++i) a[i] = a[2 * i] + a[2 * i + 1];
+        const T total = wave_tree_sum(a[0]);
+        __syncthreads();
+        return total;
+    } else if constexpr (W > 1) {
         if (c.lane == 0)
 #pragma unroll
             for (int s = 0; s < S; ++s) lds[(c.row_in_block * W + c.wave_in_row) * S + s] = seg[s];
@@ -241,6 +347,10 @@ __device__ inline T row_tree_sum(const T (&v)[S][V], T *lds, const RowCoord<W, R
         for (int i = 0; i < w / 2; ++i) seg[i] = seg[2 * i] + seg[2 * i + 1];
     return seg[0];
 }
+template <typename T, int V, int S, int W, int R, int L>
+__device__ inline T row_tree_sum(const T (&v)[S][V], T *lds, const RowCoord<W, R, L> &c) {
+    return row_tree_sum<T, V, S, W, R, L>([&](int s, int i) { return v[s][i]; }, lds, c);
+}
 
 // Plain IEEE maximum over the padded row (v_max: a NaN operand yields the
 // other one, and +0/-0 ties are unordered). Softmax uses it in place of
@@ -250,14 +360,14 @@ __device__ inline T row_tree_sum(const T (&v)[S][V], T *lds, const RowCoord<W, R
 // either rule; and a zero maximum enters only through x - m, where
 // x - (+0) and x - (-0) differ at most in the sign of a zero, which exp maps
 // to the same 1.
-template <typename T, int V, int S, int W, int R>
-__device__ inline T row_max_plain(const T (&v)[S][V], T *lds, const RowCoord<W, R> &c) {
+template <typename T, int V, int S, int W, int R, int L>
+__device__ inline T row_max_plain(const T (&v)[S][V], T *lds, const RowCoord<W, R, L> &c) {
     T x = v[0][0];
 #pragma unroll
     for (int s = 0; s < S; ++s)
 #pragma unroll
         for (int i = 0; i < V; ++i) x = vmax(x, v[s][i]);
-    x = wave_vmax(x);
+    x = lanes_vmax<L>(x);
     if constexpr (W > 1) {
         if (c.lane == 0) lds[c.row_in_block * W + c.wave_in_row] = x;
         __syncthreads();
@@ -318,33 +428,34 @@ struct RowDiv<double> {
 // The value softmax takes x - max of: element j of a row, optionally
 // as where(j <= qi, x * scale, -inf) (masked 1: causal, masked 2: scale only).
 template <typename T>
-__device__ inline T softmax_arg(T raw, int64_t j, int64_t qi, int masked, T scale) {
+__device__ inline T softmax_arg(T raw, int j, int qi, int masked, T scale) {
     if (!masked) return raw;
     const T sc = canon(raw * scale);
     return (masked == 2 || j <= qi) ? sc : neg_inf<T>();
 }
 
 // One row: v holds the raw row (padding -inf) on entry and the softmax on
-// exit; xr is the row in memory (re-read only by the rare exp fallback).
+// exit; xr is the row in memory (re-read only by the rare exp fallback, which
+// may use the result row yr as its working space).
 // FAITHFUL (binary64 only): the faithful exp and one reciprocal per row in
 // place of the correctly rounded exp and the IEEE division.
-template <typename T, int V, int S, int W, int R, bool FAITHFUL = false>
-__device__ inline void softmax_row(T (&v)[S][V], const T *__restrict__ xr, int64_t row, int64_t n, int masked,
-                                   T scale, int64_t q_len, T *lds, const RowCoord<W, R> &c,
+template <typename T, int V, int S, int W, int R, int L, bool FAITHFUL = false>
+__device__ inline void softmax_row(T (&v)[S][V], const T *xr, T *yr, int64_t row, int n, int masked, T scale,
+                                   int64_t q_len, T *lds, const RowCoord<W, R, L> &c,
                                    const typename RowExpTab<T>::type &tab) {
-    constexpr int SEG = 64 * W * V;
-    const int64_t qi = masked ? row % q_len : 0;
+    constexpr int SEG = L * W * V;
+    const int qi = masked ? (int)(row % q_len) : 0;
     if (masked) {
 #pragma unroll
         for (int s = 0; s < S; ++s)
 #pragma unroll
             for (int i = 0; i < V; ++i) {
-                const int64_t j = (int64_t)s * SEG + (int64_t)c.tid_in_row * V + i;
+                const int j = s * SEG + c.tid_in_row * V + i;
                 if (j < n) v[s][i] = softmax_arg(v[s][i], j, qi, masked, scale);
             }
     }
-    const T m = row_max_plain<T, V, S, W, R>(v, lds, c);
-    const bool full = n == (int64_t)S * SEG;
+    const T m = row_max_plain<T, V, S, W, R, L>(v, lds, c);
+    const bool full = n == S * SEG;
     if constexpr (sizeof(T) == 4) {
         // exp(x - m) in place: the branch-free fast path for every element
         // (2^(j/64) from the lane-held table), then one wave-uniform pass of
@@ -359,15 +470,45 @@ __device__ inline void softmax_row(T (&v)[S][V], const T *__restrict__ xr, int64
                 bool slow;
                 v[s][i] = expf_fast<true>(v[s][i] - m, tab, slow);
                 flagged.set(s * V + i, slow);
+                // long rows: a segment at a time, for registers
+                if (S * V > 16 && i == V - 1) __builtin_amdgcn_sched_barrier(0);
             }
-        if (flagged.any()) {
+        if constexpr (S * V <= 16) {
+            if (flagged.any()) {
+#pragma unroll
+                for (int s = 0; s < S; ++s)
+#pragma unroll
+                    for (int i = 0; i < V; ++i) {
+                        const int j = s * SEG + c.tid_in_row * V + i;
+                        if (flagged.has(s * V + i, c.lane) && (full || j < n))
+                            v[s][i] = expf_slow(softmax_arg(xr[j], j, qi, masked, scale) - m);
+                    }
+            }
+        } else if (flagged.any()) {
+            // many elements per lane: the flagged elements are finished in the
+            // result row in memory (each lane its own), where the others wait,
+            // so no register is held across the core; an element not yet
+            // finished keeps its input there when the call is in place. A
+            // call of the core per element left the row in scratch memory
+            // ([1000, 32003] binary32: 3.5 ms, 3600 bytes of it per lane).
 #pragma unroll
             for (int s = 0; s < S; ++s)
 #pragma unroll
                 for (int i = 0; i < V; ++i) {
-                    const int64_t j = (int64_t)s * SEG + (int64_t)c.tid_in_row * V + i;
-                    if (flagged.has(s * V + i, c.lane) && (full || j < n))
-                        v[s][i] = expf_slow(softmax_arg(xr[j], j, qi, masked, scale) - m);
+                    const int j = s * SEG + c.tid_in_row * V + i;
+                    if (j < n && !flagged.has(s * V + i, c.lane)) yr[j] = v[s][i];
+                }
+            while (flagged.any()) {
+                const int k = flagged.take();
+                const int j = (k / V) * SEG + c.tid_in_row * V + k % V;
+                if (k >= 0 && j < n) yr[j] = expf_cr_dd(softmax_arg(xr[j], j, qi, masked, scale) - m);
+            }
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+#pragma unroll
+                for (int i = 0; i < V; ++i) {
+                    const int j = s * SEG + c.tid_in_row * V + i;
+                    v[s][i] = j < n ? yr[j] : T(-0.0);
                 }
         }
         if (!full) {
@@ -375,11 +516,11 @@ __device__ inline void softmax_row(T (&v)[S][V], const T *__restrict__ xr, int64
             for (int s = 0; s < S; ++s)
 #pragma unroll
                 for (int i = 0; i < V; ++i) {
-                    const int64_t j = (int64_t)s * SEG + (int64_t)c.tid_in_row * V + i;
+                    const int j = s * SEG + c.tid_in_row * V + i;
                     if (j >= n) v[s][i] = T(-0.0);
                 }
         }
-        const T total = row_tree_sum<T, V, S, W, R>(v, lds, c);
+        const T total = row_tree_sum<T, V, S, W, R, L>(v, lds, c);
         if (total != total) {
             // a NaN total makes every quotient the canonical NaN
 #pragma unroll
@@ -410,11 +551,11 @@ __device__ inline void softmax_row(T (&v)[S][V], const T *__restrict__ xr, int64
             for (int s = 0; s < S; ++s)
 #pragma unroll
                 for (int i = 0; i < V; ++i) {
-                    const int64_t j = (int64_t)s * SEG + (int64_t)c.tid_in_row * V + i;
+                    const int j = s * SEG + c.tid_in_row * V + i;
                     if (j >= n) v[s][i] = T(-0.0);
                 }
         }
-        const T total = row_tree_sum<T, V, S, W, R>(v, lds, c);
+        const T total = row_tree_sum<T, V, S, W, R, L>(v, lds, c);
         if (total != total) {
 #pragma unroll
             for (int s = 0; s < S; ++s)
@@ -442,14 +583,36 @@ __device__ inline void softmax_row(T (&v)[S][V], const T *__restrict__ xr, int64
                 v[s][i] = exp_fast<true>(v[s][i] - m, tab, slow);
                 flagged.set(s * V + i, slow);
             }
-        if (flagged.any()) {
+        if constexpr (S * V <= 16) {
+            if (flagged.any()) {
+#pragma unroll
+                for (int s = 0; s < S; ++s)
+#pragma unroll
+                    for (int i = 0; i < V; ++i) {
+                        const int j = s * SEG + c.tid_in_row * V + i;
+                        if (flagged.has(s * V + i, c.lane) && (full || j < n))
+                            v[s][i] = exp_slow64(softmax_arg(xr[j], j, qi, masked, scale) - m);
+                    }
+            }
+        } else if (flagged.any()) {
 #pragma unroll
             for (int s = 0; s < S; ++s)
 #pragma unroll
                 for (int i = 0; i < V; ++i) {
-                    const int64_t j = (int64_t)s * SEG + (int64_t)c.tid_in_row * V + i;
-                    if (flagged.has(s * V + i, c.lane) && (full || j < n))
-                        v[s][i] = exp_slow64(softmax_arg(xr[j], j, qi, masked, scale) - m);
+                    const int j = s * SEG + c.tid_in_row * V + i;
+                    if (j < n && !flagged.has(s * V + i, c.lane)) yr[j] = v[s][i];
+                }
+            while (flagged.any()) {
+                const int k = flagged.take();
+                const int j = (k / V) * SEG + c.tid_in_row * V + k % V;
+                if (k >= 0 && j < n) yr[j] = exp_cr_slow(softmax_arg(xr[j], j, qi, masked, scale) - m);
+            }
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+#pragma unroll
+                for (int i = 0; i < V; ++i) {
+                    const int j = s * SEG + c.tid_in_row * V + i;
+                    v[s][i] = j < n ? yr[j] : T(-0.0);
                 }
         }
         if (!full) {
@@ -457,11 +620,11 @@ __device__ inline void softmax_row(T (&v)[S][V], const T *__restrict__ xr, int64
             for (int s = 0; s < S; ++s)
 #pragma unroll
                 for (int i = 0; i < V; ++i) {
-                    const int64_t j = (int64_t)s * SEG + (int64_t)c.tid_in_row * V + i;
+                    const int j = s * SEG + c.tid_in_row * V + i;
                     if (j >= n) v[s][i] = T(-0.0);
                 }
         }
-        const RowDiv<T> div(canon(row_tree_sum<T, V, S, W, R>(v, lds, c)));
+        const RowDiv<T> div(canon(row_tree_sum<T, V, S, W, R, L>(v, lds, c)));
 #pragma unroll
         for (int s = 0; s < S; ++s)
 #pragma unroll
@@ -474,101 +637,157 @@ __device__ inline void softmax_row(T (&v)[S][V], const T *__restrict__ xr, int64
 // common case (no mask, row length equal to the register capacity S*64W*V,
 // 16-byte aligned rows) with every bound test folded away. FAITHFUL as for
 // softmax_row.
-template <typename T, int V, int S, int W, int R, bool DENSE, bool FAITHFUL = false>
-__global__ __launch_bounds__(64 * W * R) void softmax_kernel(const T *__restrict__ x, T *__restrict__ y,
-                                                              int64_t rows, int64_t n_arg, int64_t ldx, int64_t ldy,
-                                                              bool vec_ok_arg, int masked_arg, T scale,
-                                                              int64_t q_len) {
+template <typename T, int V, int S, int W, int R, int L, bool DENSE, bool RAGGED, bool FAITHFUL = false>
+__global__ __launch_bounds__(64 * W * R, W == 16 && S == 8 && (sizeof(T) == 4 || FAITHFUL) ? 8 : 1) void softmax_kernel(const T *x, T *y,
+                                                              int64_t rows, int n_arg, int64_t ldx, int64_t ldy,
+                                                              int masked_arg, T scale, int64_t q_len) {
     __shared__ T lds[R * W * S];
-    constexpr int SEG = 64 * W * V;
-    const int64_t n = DENSE ? (int64_t)S * SEG : n_arg;
-    const bool vec_ok = DENSE || vec_ok_arg;
+    constexpr int SEG = L * W * V;
+    const int n = DENSE ? S * SEG : n_arg;
     const int masked = DENSE ? 0 : masked_arg;
     __shared__ double2 exp_tab[sizeof(T) == 8 ? 64 : 1];
     if constexpr (sizeof(T) == 8) {
         if (threadIdx.x < 64) exp_tab[threadIdx.x] = double2{chelis_exp2_64_tab[threadIdx.x][0], chelis_exp2_64_tab[threadIdx.x][1]};
         __syncthreads();
     }
-    RowCoord<W, R> c;
-    if (c.row >= rows) return;  // whole row groups exit together (R rows per block, W waves each)
+    RowCoord<W, R, L> c(rows);
+    if (L == 64 && !c.live) return;  // whole row groups exit together (R rows per block, W waves each)
     const T *xr = x + c.row * ldx;
     const typename RowExpTab<T>::type tab = RowExpTab<T>::make(c.lane, exp_tab);
     T v[S][V];
     // causal rows read only j <= qi: the mask turns every later element into
     // -inf whatever it holds, which is the padding value
-    const int64_t n_load = masked == 1 ? (c.row % q_len + 1 < n ? c.row % q_len + 1 : n) : n;
-    load_row<T, V, S, W>(xr, n_load, vec_ok, c.tid_in_row, neg_inf<T>(), v);
-    softmax_row<T, V, S, W, R, FAITHFUL>(v, xr, c.row, n, masked, scale, q_len, lds, c, tab);
-    store_row<T, V, S, W>(y + c.row * ldy, n, vec_ok, c.tid_in_row, v);
+    if constexpr (DENSE) {
+        load_dense<T, V, S, W, L>(xr, c.tid_in_row, v);
+    } else {
+        const int need = masked == 1 ? (int)(c.row % q_len) + 1 : n, up = (need + V - 1) / V * V;
+        const int n_load = up < n ? up : n;
+        RowLoad<T, V, S, W, L, RAGGED> lx(xr, n_load, c.tid_in_row);
+        lx.issue();
+        lx.take(neg_inf<T>(), v);
+    }
+    softmax_row<T, V, S, W, R, L, FAITHFUL>(v, xr, y + c.row * ldy, c.row, n, masked, scale, q_len, lds, c, tab);
+    if (c.live) store_row<T, V, S, W, L, RAGGED>(y + c.row * ldy, n, c.tid_in_row, v);
 }
 
-// dx = y * (g - sum(g * y)) over the last axis.
-template <typename T, int V, int S, int W, int R>
+// dx = y * (g - sum(g * y)) over the last axis. Rows of sixteen segments
+// (two of them are more than a lane's registers) are read again for the
+// second half, from the caches where they fit.
+template <typename T, int V, int S, int W, int R, int L, bool RAGGED>
 __global__ __launch_bounds__(64 * W * R) void softmax_adjoint_kernel(const T *__restrict__ y,
                                                                       const T *__restrict__ g, T *__restrict__ dx,
-                                                                      int64_t rows, int64_t n, int64_t ldy,
-                                                                      int64_t ldg, int64_t ldd, bool vec_ok) {
+                                                                      int64_t rows, int n, int64_t ldy,
+                                                                      int64_t ldg, int64_t ldd) {
     __shared__ T lds[R * W * S];
-    RowCoord<W, R> c;
-    if (c.row >= rows) return;
-    T yv[S][V], gv[S][V], t[S][V];
-    load_row<T, V, S, W>(y + c.row * ldy, n, vec_ok, c.tid_in_row, T(-0.0), yv);
-    load_row<T, V, S, W>(g + c.row * ldg, n, vec_ok, c.tid_in_row, T(-0.0), gv);
-    constexpr int SEG = 64 * W * V;
+    RowCoord<W, R, L> c(rows);
+    if (L == 64 && !c.live) return;
+    constexpr int SEG = L * W * V;
+    const T *yr = y + c.row * ldy, *gr = g + c.row * ldg;
+    T *dr = dx + c.row * ldd;
+    auto product = [](T a, T b) { return canon(a * b); };
+    if constexpr (S < 16) {
+        T yv[S][V], gv[S][V];
+        RowLoad<T, V, S, W, L, RAGGED> ly(yr, n, c.tid_in_row), lg(gr, n, c.tid_in_row);
+        ly.issue();
+        lg.issue();
+        ly.take(T(-0.0), yv);
+        lg.take(T(-0.0), gv);
+        const T total = canon(row_tree_sum<T, V, S, W, R, L>(
+            [&](int s, int i) {
+                return s * SEG + c.tid_in_row * V + i < n ? product(gv[s][i], yv[s][i]) : T(-0.0);
+            },
+            lds, c));
 #pragma unroll
-    for (int s = 0; s < S; ++s)
+        for (int s = 0; s < S; ++s)
 #pragma unroll
-        for (int i = 0; i < V; ++i) {
-            const int64_t j = (int64_t)s * SEG + (int64_t)c.tid_in_row * V + i;
-            t[s][i] = (j < n) ? canon(gv[s][i] * yv[s][i]) : T(-0.0);
-        }
-    const T total = canon(row_tree_sum<T, V, S, W, R>(t, lds, c));
+            for (int i = 0; i < V; ++i) gv[s][i] = canon(yv[s][i] * canon(gv[s][i] - total));
+        if (c.live) store_row<T, V, S, W, L, RAGGED>(dr, n, c.tid_in_row, gv);
+    } else {
+        // in place (dx is y or g) is safe: every read of the row precedes
+        // the barrier below or is of the lane's own elements
+        T t[S][V];
 #pragma unroll
-    for (int s = 0; s < S; ++s)
+        for (int s = 0; s < S; ++s)
 #pragma unroll
-        for (int i = 0; i < V; ++i) t[s][i] = canon(yv[s][i] * canon(gv[s][i] - total));
-    store_row<T, V, S, W>(dx + c.row * ldd, n, vec_ok, c.tid_in_row, t);
+            for (int i = 0; i < V; ++i) {
+                const int j = s * SEG + c.tid_in_row * V + i;
+                t[s][i] = j < n ? product(gr[j], yr[j]) : T(-0.0);
+            }
+        const T total = canon(row_tree_sum<T, V, S, W, R, L>(t, lds, c));
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+#pragma unroll
+            for (int i = 0; i < V; ++i) {
+                const int j = s * SEG + c.tid_in_row * V + i;
+                if (j < n) dr[j] = canon(yr[j] * canon(gr[j] - total));
+            }
+    }
 }
 
 // layer_norm: mean = tree(x)/n; c = x - mean; var = tree(c*c)/n;
 // y = (c / sqrt(var + eps)) * gamma + beta, every primitive finalized.
-template <typename T, int V, int S, int W, int R>
+template <typename T, int V, int S, int W, int R, int L, bool RAGGED>
 __global__ __launch_bounds__(64 * W * R) void layer_norm_kernel(const T *__restrict__ x, const T *__restrict__ gamma,
                                                                  const T *__restrict__ beta, T *__restrict__ y,
-                                                                 int64_t rows, int64_t n, int64_t ldx, int64_t ldy,
-                                                                 bool vec_ok, T eps) {
+                                                                 int64_t rows, int n, int64_t ldx, int64_t ldy,
+                                                                 T eps) {
     __shared__ T lds[R * W * S];
-    RowCoord<W, R> c;
-    if (c.row >= rows) return;
-    T v[S][V], q[S][V], gm[S][V], bt[S][V];
-    load_row<T, V, S, W>(x + c.row * ldx, n, vec_ok, c.tid_in_row, T(-0.0), v);
+    RowCoord<W, R, L> c(rows);
+    if (L == 64 && !c.live) return;
     // gamma/beta are [n] vectors shared by every row: their loads go out with
     // the row's, ahead of the reductions' barriers (after them each row waited
-    // out two more cache round trips: [65536,1024] 90.8 -> 88.5 us)
-    load_row<T, V, S, W, false>(gamma, n, vec_ok, c.tid_in_row, T(0), gm);
-    load_row<T, V, S, W, false>(beta, n, vec_ok, c.tid_in_row, T(0), bt);
+    // out two more cache round trips: [65536,1024] 90.8 -> 88.5 us); rows of
+    // sixteen waves have no registers to hold them that long
+    constexpr bool EARLY = sizeof(T) == 4 ? S * W < 128 : S < 8;
+    T v[S][V], gm[EARLY ? S : 1][V], bt[EARLY ? S : 1][V];
+    RowLoad<T, V, S, W, L, RAGGED> lx(x + c.row * ldx, n, c.tid_in_row);
+    if constexpr (EARLY) {
+        RowLoad<T, V, S, W, L, RAGGED, false, false> lg(gamma, n, c.tid_in_row), lb(beta, n, c.tid_in_row);
+        lx.issue();
+        lg.issue();
+        lb.issue();
+        lx.take(T(-0.0), v);
+        lg.take(T(0), gm);
+        lb.take(T(0), bt);
+    } else {
+        lx.issue();
+        lx.take(T(-0.0), v);
+    }
     const T extent = (T)n;
-    const T mean = canon(canon(row_tree_sum<T, V, S, W, R>(v, lds, c)) / extent);
-    constexpr int SEG = 64 * W * V;
+    const T mean = canon(canon(row_tree_sum<T, V, S, W, R, L>(v, lds, c)) / extent);
+    constexpr int SEG = L * W * V;
 #pragma unroll
     for (int s = 0; s < S; ++s)
 #pragma unroll
-        for (int i = 0; i < V; ++i) {
-            const int64_t j = (int64_t)s * SEG + (int64_t)c.tid_in_row * V + i;
-            v[s][i] = canon(v[s][i] - mean);
-            q[s][i] = (j < n) ? canon(v[s][i] * v[s][i]) : T(-0.0);
-        }
-    const T var = canon(canon(row_tree_sum<T, V, S, W, R>(q, lds, c)) / extent);
+        for (int i = 0; i < V; ++i) v[s][i] = canon(v[s][i] - mean);
+    const T var = canon(canon(row_tree_sum<T, V, S, W, R, L>(
+                            [&](int s, int i) {
+                                return s * SEG + c.tid_in_row * V + i < n ? canon(v[s][i] * v[s][i]) : T(-0.0);
+                            },
+                            lds, c)) /
+                        extent);
     const T denom = canon_bits(sqrt(canon(var + eps)));
 #pragma unroll
-    for (int s = 0; s < S; ++s)
+    for (int s = 0; s < S; ++s) {
+        if constexpr (EARLY) {
 #pragma unroll
-        for (int i = 0; i < V; ++i) v[s][i] = canon(canon(v[s][i] / denom) * gm[s][i]);
+            for (int i = 0; i < V; ++i) v[s][i] = canon(canon(v[s][i] / denom) * gm[s][i]);
 #pragma unroll
-    for (int s = 0; s < S; ++s)
+            for (int i = 0; i < V; ++i) v[s][i] = canon(v[s][i] + bt[s][i]);
+        } else {
+            T gs[1][V], bs[1][V];
+            const int off = s * SEG < n ? s * SEG : 0;
+            RowLoad<T, V, 1, W, L, RAGGED, false, false> lg(gamma + off, n - off, c.tid_in_row), lb(beta + off, n - off, c.tid_in_row);
+            lg.issue();
+            lb.issue();
+            lg.take(T(0), gs);
+            lb.take(T(0), bs);
 #pragma unroll
-        for (int i = 0; i < V; ++i) v[s][i] = canon(v[s][i] + bt[s][i]);
-    store_row<T, V, S, W>(y + c.row * ldy, n, vec_ok, c.tid_in_row, v);
+            for (int i = 0; i < V; ++i) v[s][i] = canon(canon(canon(v[s][i] / denom) * gs[0][i]) + bs[0][i]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    if (c.live) store_row<T, V, S, W, L, RAGGED>(y + c.row * ldy, n, c.tid_in_row, v);
 }
 
 // ---------------------------------------------------------------- dispatch
@@ -579,54 +798,52 @@ struct RowArgs {
     const void *a, *b, *c;
     void *out;
     int64_t rows, n, lda, ldb, ldo;
-    bool vec_ok;
     int masked;
     double scale;
     int64_t q_len;
     double eps;
 };
 
-template <typename T, int V, int S, int W, int R>
+template <typename T, int V, int S, int W, int R, int L, bool DENSE, bool RAGGED>
+void launch_softmax(const RowArgs &a, unsigned grid, hipStream_t st) {
+    const dim3 block(64 * W * R);
+    // binary64 outside the exact mode: the faithful row
+    if constexpr (sizeof(T) == 8) {
+        if (!exact_mode()) {
+            softmax_kernel<T, V, S, W, R, L, DENSE, RAGGED, true><<<grid, block, 0, st>>>(
+                (const T *)a.a, (T *)a.out, a.rows, (int)a.n, a.lda, a.ldo, a.masked, (T)a.scale, a.q_len);
+            return;
+        }
+    }
+    softmax_kernel<T, V, S, W, R, L, DENSE, RAGGED><<<grid, block, 0, st>>>(
+        (const T *)a.a, (T *)a.out, a.rows, (int)a.n, a.lda, a.ldo, a.masked, (T)a.scale, a.q_len);
+}
+
+template <typename T, int V, int S, int W, int R, int L, bool RAGGED>
+void launch_pair(RowOp op, const RowArgs &a, unsigned grid, hipStream_t st) {
+    const dim3 block(64 * W * R);
+    if (op == RowOp::SoftmaxAdjoint)
+        softmax_adjoint_kernel<T, V, S, W, R, L, RAGGED><<<grid, block, 0, st>>>(
+            (const T *)a.a, (const T *)a.b, (T *)a.out, a.rows, (int)a.n, a.lda, a.ldb, a.ldo);
+    else
+        layer_norm_kernel<T, V, S, W, R, L, RAGGED><<<grid, block, 0, st>>>(
+            (const T *)a.a, (const T *)a.b, (const T *)a.c, (T *)a.out, a.rows, (int)a.n, a.lda, a.ldo, (T)a.eps);
+}
+
+template <typename T, int V, int S, int W, int R, int L>
 int32_t launch_shape(RowOp op, const RowArgs &a, hipStream_t st) {
-    const unsigned grid = grid_for(a.rows, R);
+    const unsigned grid = grid_for(a.rows, R * (64 / L));
     if (!grid_fits(grid, 64 * W * R)) return set_error(CHELIS_HIP_EUNSUPPORTED, "rows: %lld rows exceed one launch",
                                                        (long long)a.rows);
-    const dim3 block(64 * W * R);
-    switch (op) {
-        case RowOp::Softmax: {
-            const bool dense = !a.masked && a.vec_ok && a.n == (int64_t)S * 64 * W * V;
-            // binary64 outside the exact mode: the faithful row
-            if constexpr (sizeof(T) == 8) {
-                if (!exact_mode()) {
-                    if (dense)
-                        softmax_kernel<T, V, S, W, R, true, true><<<grid, block, 0, st>>>(
-                            (const T *)a.a, (T *)a.out, a.rows, a.n, a.lda, a.ldo, a.vec_ok, a.masked, (T)a.scale,
-                            a.q_len);
-                    else
-                        softmax_kernel<T, V, S, W, R, false, true><<<grid, block, 0, st>>>(
-                            (const T *)a.a, (T *)a.out, a.rows, a.n, a.lda, a.ldo, a.vec_ok, a.masked, (T)a.scale,
-                            a.q_len);
-                    break;
-                }
-            }
-            if (dense) {
-                softmax_kernel<T, V, S, W, R, true><<<grid, block, 0, st>>>(
-                    (const T *)a.a, (T *)a.out, a.rows, a.n, a.lda, a.ldo, a.vec_ok, a.masked, (T)a.scale, a.q_len);
-            } else {
-                softmax_kernel<T, V, S, W, R, false><<<grid, block, 0, st>>>(
-                    (const T *)a.a, (T *)a.out, a.rows, a.n, a.lda, a.ldo, a.vec_ok, a.masked, (T)a.scale, a.q_len);
-            }
-            break;
-        }
-        case RowOp::SoftmaxAdjoint:
-            softmax_adjoint_kernel<T, V, S, W, R><<<grid, block, 0, st>>>(
-                (const T *)a.a, (const T *)a.b, (T *)a.out, a.rows, a.n, a.lda, a.ldb, a.ldo, a.vec_ok);
-            break;
-        case RowOp::LayerNorm:
-            layer_norm_kernel<T, V, S, W, R><<<grid, block, 0, st>>>(
-                (const T *)a.a, (const T *)a.b, (const T *)a.c, (T *)a.out, a.rows, a.n, a.lda, a.ldo, a.vec_ok,
-                (T)a.eps);
-            break;
+    const bool ragged = a.n % V != 0;
+    if (op == RowOp::Softmax) {
+        if (ragged) launch_softmax<T, V, S, W, R, L, false, true>(a, grid, st);
+        else if (!a.masked && a.n == (int64_t)S * L * W * V) launch_softmax<T, V, S, W, R, L, true, false>(a, grid, st);
+        else launch_softmax<T, V, S, W, R, L, false, false>(a, grid, st);
+    } else if (ragged) {
+        launch_pair<T, V, S, W, R, L, true>(op, a, grid, st);
+    } else {
+        launch_pair<T, V, S, W, R, L, false>(op, a, grid, st);
     }
     CHELIS_LAUNCH_CHECK();
     return CHELIS_HIP_OK;
@@ -640,8 +857,14 @@ int32_t launch_rows(RowOp op, const RowArgs &a) {
     if (!st) return set_error(CHELIS_HIP_EHIP, "no HIP device");
     const int64_t seg1 = 64 * V;  // one wave, one segment
     const int64_t n = a.n;
-    if (n <= seg1) return launch_shape<T, V, 1, 1, 4>(op, a, st);
-    if (n <= 2 * seg1) return launch_shape<T, V, 2, 1, 4>(op, a, st);
+    // rows of at most half a wave's vectors: four rows per wave, sixteen lanes
+    // each (one row per wave leaves most lanes idle: softmax and adjoint of
+    // [363636, 33] binary32 206 -> 65 us, [120000, 100] 84 -> 48; layer norm
+    // 118 -> 36 and 49 -> 23)
+    if (n <= 16 * V) return launch_shape<T, V, 1, 1, 4, 16>(op, a, st);
+    if (n <= 32 * V) return launch_shape<T, V, 2, 1, 4, 16>(op, a, st);
+    if (n <= seg1) return launch_shape<T, V, 1, 1, 4, 64>(op, a, st);
+    if (n <= 2 * seg1) return launch_shape<T, V, 2, 1, 4, 64>(op, a, st);
     // binary32 rows of 513-1024: two waves per row, two segments each
     // (23.4 against 24.2 us for [16384, 1024] with one wave of four
     // segments, same box: the shorter per-wave dependency chain keeps more
@@ -649,15 +872,19 @@ int32_t launch_rows(RowOp op, const RowArgs &a) {
     // block, so blocks retire independently and the waves of a CU drift
     // apart, one wave's loads overlapping another's arithmetic
     if (n <= 4 * seg1) {
-        if constexpr (sizeof(T) == 4) return launch_shape<T, V, 2, 2, 1>(op, a, st);
-        return launch_shape<T, V, 4, 1, 1>(op, a, st);
+        if constexpr (sizeof(T) == 4) return launch_shape<T, V, 2, 2, 1, 64>(op, a, st);
+        if (op == RowOp::LayerNorm) return launch_shape<T, V, 4, 1, 4, 64>(op, a, st);
+        return launch_shape<T, V, 4, 1, 1, 64>(op, a, st);
     }
-    if (n <= 8 * seg1) return launch_shape<T, V, 8, 1, 2>(op, a, st);
-    if (n <= 16 * seg1) return launch_shape<T, V, 4, 4, 1>(op, a, st);
-    if (n <= 32 * seg1) return launch_shape<T, V, 8, 4, 1>(op, a, st);
-    if (n <= 64 * seg1) return launch_shape<T, V, 8, 8, 1>(op, a, st);
-    if (n <= 128 * seg1) return launch_shape<T, V, 8, 16, 1>(op, a, st);
-    if (n <= 256 * seg1) return launch_shape<T, V, 16, 16, 1>(op, a, st);
+    // binary64 layer norm: two waves (gamma and beta fit beside the row;
+    // [23391, 513] 64.4 -> 60.9 us)
+    if (n <= 8 * seg1 && sizeof(T) == 8 && op == RowOp::LayerNorm) return launch_shape<T, V, 4, 2, 1, 64>(op, a, st);
+    if (n <= 8 * seg1) return launch_shape<T, V, 8, 1, 2, 64>(op, a, st);
+    if (n <= 16 * seg1) return launch_shape<T, V, 4, 4, 1, 64>(op, a, st);
+    if (n <= 32 * seg1) return launch_shape<T, V, 8, 4, 1, 64>(op, a, st);
+    if (n <= 64 * seg1) return launch_shape<T, V, 8, 8, 1, 64>(op, a, st);
+    if (n <= 128 * seg1) return launch_shape<T, V, 8, 16, 1, 64>(op, a, st);
+    if (n <= 256 * seg1) return launch_shape<T, V, 16, 16, 1, 64>(op, a, st);
     return set_error(CHELIS_HIP_EUNSUPPORTED, "row length %lld exceeds the in-register row capacity %lld",
                      (long long)n, (long long)(256 * seg1));
 }
@@ -666,8 +893,6 @@ int32_t dispatch(chelis_dtype dt, RowOp op, const RowArgs &a) {
     if (a.rows == 0 || a.n == 0) return CHELIS_HIP_OK;
     return dt == CHELIS_DTYPE_F32 ? launch_rows<float>(op, a) : launch_rows<double>(op, a);
 }
-
-bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 int32_t check_rows_pair(const chelis_gpu_tensor *x, const chelis_gpu_tensor *y, RowView *vx, RowView *vy,
                         const char *what) {
@@ -826,9 +1051,7 @@ extern "C" int32_t chelis_hip_softmax(const chelis_gpu_tensor *x, const chelis_g
     RowView vx, vy;
     if (int32_t s = check_rows_pair(x, y, &vx, &vy, "softmax")) return s;
     if (vx.rows && long_rows(x->dtype, vx.n)) return long_softmax(x, y, vx, vy);
-    const int64_t V = 16 / dtype_width(x->dtype);
-    RowArgs a{x->data, nullptr, nullptr, y->data, vx.rows, vx.n, vx.ld, 0, vy.ld,
-              aligned16(x->data) && aligned16(y->data) && vx.ld % V == 0 && vy.ld % V == 0, 0, 1.0, 1, 0.0};
+    RowArgs a{x->data, nullptr, nullptr, y->data, vx.rows, vx.n, vx.ld, 0, vy.ld, 0, 1.0, 1, 0.0};
     return dispatch(x->dtype, RowOp::Softmax, a);
 }
 
@@ -840,10 +1063,7 @@ extern "C" int32_t chelis_hip_scaled_masked_softmax(const chelis_gpu_tensor *x, 
     const int64_t q_len = x->shape[x->rank - 2];
     if (causal && q_len != vx.n)
         return set_error(CHELIS_HIP_EDOMAIN, "scaled_masked_softmax: causal mask needs square score matrices");
-    const int64_t V = 16 / dtype_width(x->dtype);
-    RowArgs a{x->data, nullptr, nullptr, y->data, vx.rows, vx.n, vx.ld, 0, vy.ld,
-              aligned16(x->data) && aligned16(y->data) && vx.ld % V == 0 && vy.ld % V == 0,
-              causal ? 1 : 2, scale, q_len > 0 ? q_len : 1, 0.0};
+    RowArgs a{x->data, nullptr, nullptr, y->data, vx.rows, vx.n, vx.ld, 0, vy.ld, causal ? 1 : 2, scale, q_len > 0 ? q_len : 1, 0.0};
     return dispatch(x->dtype, RowOp::Softmax, a);
 }
 
@@ -855,11 +1075,7 @@ extern "C" int32_t chelis_hip_softmax_adjoint(const chelis_gpu_tensor *y, const 
     if (g->dtype != y->dtype || !same_shape(g, y) || !row_view(g, &vg))
         return set_error(CHELIS_HIP_EDOMAIN, "softmax_adjoint: g must match y");
     if (vy.rows && long_rows(y->dtype, vy.n)) return long_softmax_adjoint(y, g, dx, vy, vg, vd);
-    const int64_t V = 16 / dtype_width(y->dtype);
-    RowArgs a{y->data, g->data, nullptr, dx->data, vy.rows, vy.n, vy.ld, vg.ld, vd.ld,
-              aligned16(y->data) && aligned16(g->data) && aligned16(dx->data) && vy.ld % V == 0 &&
-                  vg.ld % V == 0 && vd.ld % V == 0,
-              0, 1.0, 1, 0.0};
+    RowArgs a{y->data, g->data, nullptr, dx->data, vy.rows, vy.n, vy.ld, vg.ld, vd.ld, 0, 1.0, 1, 0.0};
     return dispatch(y->dtype, RowOp::SoftmaxAdjoint, a);
 }
 
@@ -875,10 +1091,6 @@ extern "C" int32_t chelis_hip_layer_norm(const chelis_gpu_tensor *x, const cheli
             return set_error(CHELIS_HIP_EDOMAIN, "layer_norm: gamma/beta must be contiguous [hidden]");
     if (vx.n == 0) return set_error(CHELIS_HIP_EDOMAIN, "layer_norm: hidden extent must be positive");
     if (vx.rows && long_rows(x->dtype, vx.n)) return long_layer_norm(x, gamma, beta, epsilon, y, vx, vy);
-    const int64_t V = 16 / dtype_width(x->dtype);
-    RowArgs a{x->data, gamma->data, beta->data, y->data, vx.rows, vx.n, vx.ld, 0, vy.ld,
-              aligned16(x->data) && aligned16(y->data) && aligned16(gamma->data) && aligned16(beta->data) &&
-                  vx.ld % V == 0 && vy.ld % V == 0,
-              0, 1.0, 1, epsilon};
+    RowArgs a{x->data, gamma->data, beta->data, y->data, vx.rows, vx.n, vx.ld, 0, vy.ld, 0, 1.0, 1, epsilon};
     return dispatch(x->dtype, RowOp::LayerNorm, a);
 }

@@ -198,6 +198,68 @@ def test_softmax_adjoint(dtype, n):
     assert bits_equal(dx, O.softmax_adjoint_rows(yv, g))
 
 
+ROW_EDGES = [1, 2, 3, 4, 5, 31, 32, 33, 63, 64, 65, 127, 128, 129, 255, 257, 511, 513, 1023, 1025, 2047, 4095, 4097,
+             8191, 16383, 16385, 32003, 32767, 32768]
+
+
+@pytest.mark.parametrize("n", ROW_EDGES + [65535])
+def test_row_shapes_at_the_edges_f32(n):
+    """Every register shape's first and last row length, rows that start off a
+    16-byte boundary (one element in, an odd row stride), a row count that
+    fills no workgroup, and the result in place: bit-exact."""
+    rng, rows, ld = np.random.default_rng(n), 7, n + 1 + n % 2
+    def held(scale=1.0):
+        a = (rng.standard_normal((rows, n)) * scale).astype(np.float32)
+        flat = np.zeros(rows * ld + 1, np.float32)
+        np.lib.stride_tricks.as_strided(flat[1:], (rows, n), (4 * ld, 4))[:] = a
+        d = C.to_device(flat)
+        return a, d.view((rows, n), (ld, 1), 1)
+    # a wide spread: some exps land where the fast path asks for the full one
+    x, dx = held(20.0)
+    x[0, 0] = 0.0
+    ref = O.softmax_rows(x)
+    dx = C.to_device(np.concatenate([[0], np.pad(x, ((0, 0), (0, ld - n))).ravel()]).astype(np.float32)).view(
+        (rows, n), (ld, 1), 1)
+    out = C.empty((rows, n), np.float32)
+    C.softmax(dx, out)
+    assert bits_equal(out.numpy(), ref), mismatch_report(out.numpy(), ref)
+    C.softmax(dx, dx)
+    assert bits_equal(dx.numpy(), ref)
+    y, dy = held()
+    g, dg = held()
+    adj = O.softmax_adjoint_rows(y, g)
+    C.softmax_adjoint(dy, dg, dg)
+    assert bits_equal(dg.numpy(), adj), mismatch_report(dg.numpy(), adj)
+    gamma, beta = rng.standard_normal(n + 1).astype(np.float32), rng.standard_normal(n + 1).astype(np.float32)
+    gv, bv = (C.to_device(a).view((n,), (1,), 1) for a in (gamma, beta))
+    ln = O.layer_norm_rows(y, gamma[1:], beta[1:], np.float32(1e-5))
+    C.layer_norm(dy, gv, bv, 1e-5, dy)
+    assert bits_equal(dy.numpy(), ln), mismatch_report(dy.numpy(), ln)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 31, 32, 33, 63, 65, 127, 129, 257, 513, 1025, 2049, 8193, 16384, 16385, 32767])
+def test_row_shapes_at_the_edges_f64(n):
+    """The same in binary64: softmax bit-exact in the exact mode (the rows of
+    many segments finish their flagged exps in the result row) and within the
+    default row's bound, adjoint and layer norm bit-exact."""
+    rng, rows = np.random.default_rng(n), 5
+    x = rng.uniform(-700.0, 0.0, (rows, n))
+    x[:, 0] = 0.0
+    x[0, : n // 2] = -745.0  # subnormal exps: the full path
+    ref = O.softmax_rows(x)
+    with exact_mode():
+        d = C.to_device(x)
+        C.softmax(d, d)
+    assert bits_equal(d.numpy(), ref), mismatch_report(d.numpy(), ref)
+    assert_f64_rows_close(C.softmax(C.to_device(x)).numpy(), ref)
+    y, g = rng.standard_normal((rows, n)), rng.standard_normal((rows, n))
+    assert bits_equal(C.softmax_adjoint(C.to_device(y), C.to_device(g)).numpy(), O.softmax_adjoint_rows(y, g))
+    gamma, beta = rng.standard_normal(n), rng.standard_normal(n)
+    got = C.layer_norm(C.to_device(y), C.to_device(gamma), C.to_device(beta), 1e-5).numpy()
+    assert bits_equal(got, O.layer_norm_rows(y, gamma, beta, 1e-5))
+
+
+
 @pytest.mark.parametrize("dtype,shape", [(np.float32, (4096, 1024)), (np.float32, (100, 333)),
                                          (np.float64, (512, 1024))])
 def test_layer_norm_bit_exact(dtype, shape):
