@@ -316,6 +316,26 @@ __device__ inline void store_nt16(T *p, const typename Vec16F<T>::type &q) {
     __builtin_nontemporal_store(e, reinterpret_cast<E *>(p));
 }
 
+// The same vectors at any element-aligned address (a 16-byte global access
+// needs no more on gfx950); NT as above.
+template <bool NT, typename T>
+__device__ inline typename Vec16F<T>::type load_any16(const T *p) {
+    typedef T E __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
+    E e;
+    if constexpr (NT) e = __builtin_nontemporal_load(reinterpret_cast<const E *>(p));
+    else e = *reinterpret_cast<const E *>(p);
+    typename Vec16F<T>::type q;
+    __builtin_memcpy(&q, &e, 16);
+    return q;
+}
+template <typename T>
+__device__ inline void store_any16(T *p, const typename Vec16F<T>::type &q) {
+    typedef T E __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
+    E e;
+    __builtin_memcpy(&e, &q, 16);
+    __builtin_nontemporal_store(e, reinterpret_cast<E *>(p));
+}
+
 template <typename T, int V>
 __device__ inline void apply_step_vec(uint8_t op, const T (&x)[V], const T (&y)[V], double imm, T (&r)[V]) {
     switch (op) {
@@ -353,10 +373,14 @@ __device__ inline void apply_step_vec(uint8_t op, const T (&x)[V], const T (&y)[
 // The vector form of run_chain: V elements per thread, slots slot-major
 // ([n_in + n_steps][256] 16-byte vectors, adjacent lanes on adjacent
 // words), one op dispatch per step. r holds the last step's values.
+// Only the steps of `run` (bit per step) are evaluated: the others keep what
+// an earlier evaluation left in their slots.
 template <typename T, int V, typename Q>
-__device__ inline void run_chain_vec(const ChainDev &ch, Q *slots, int n_in, int tid, T (&r)[V]) {
+__device__ inline void run_chain_vec(const ChainDev &ch, Q *slots, int n_in, int tid, T (&r)[V],
+                                     uint32_t run = ~0u) {
 #pragma unroll 1
     for (int st = 0; st < ch.n_steps; ++st) {
+        if (!((run >> st) & 1u)) continue;
         const int a0 = ch.a0[st], a1 = ch.a1[st];
         const Q xq = slots[(a0 >= 0 ? a0 : n_in - a0 - 1) * 256 + tid];
         const Q yq = slots[(a1 >= 0 ? a1 : n_in - a1 - 1) * 256 + tid];

@@ -256,6 +256,97 @@ __global__ __launch_bounds__(256) void fused_flat_vec_kernel(ChainDev ch, FlatGr
     }
 }
 
+// ---------------------------------------------------------------- broadcast maps
+// Operands that run with the output along its last axis or are one element
+// of it (stride 1 or 0 there), any strides on the axes before: row and
+// column broadcasts. A thread owns V = 16 / sizeof(T) consecutive columns
+// (any alignment, the last of a row's vectors in part) of R rows, the rows
+// of one pass over the grid next to each other so a wave's accesses are
+// contiguous whatever the row length. The next row's loads are in flight
+// while the interpreter runs this one's. What depends on the column alone
+// (an operand with no stride before the last axis, and the steps over such
+// operands and constants: a column's scale, say) is loaded and evaluated for
+// the first row and kept in its slots for the others.
+// ([16384,4096] f32, (x - mean[col]) / sqrt(var[col] + eps): 528 us one
+// element per interpreter run.)
+struct RowMap {
+    int64_t rows, last, groups;  // groups: rows per pass, ceil(rows / R)
+    uint32_t nv, R;              // vectors per row, rows per thread
+    uint32_t splat, column;      // bit k: input k has one element per row / depends on the column alone
+    uint32_t step_column;        // bit s: step s depends on the column alone
+    Shape outer;                 // the axes before the last
+};
+
+template <typename T>
+__global__ __launch_bounds__(256) void fused_rows_kernel(ChainDev ch, Operands ops, RowMap m, T *out) {
+    constexpr int V = 16 / sizeof(T), NI = CHELIS_FUSED_MAX_INPUTS;
+    using Q = typename Vec16F<T>::type;
+    extern __shared__ __align__(16) unsigned char rows_lds[];
+    Q *slots = reinterpret_cast<Q *>(rows_lds);
+    const int64_t id = (int64_t)blockIdx.x * kMapThreads + threadIdx.x;
+    const int64_t g = id / m.nv;
+    if (g >= m.groups) return;
+    const int64_t c0 = (id - g * m.nv) * V;
+    const bool full = c0 + V <= m.last;
+    Q in[NI];
+    auto load = [&](int64_t row, bool first) {
+        int64_t off[NI];
+#pragma unroll
+        for (int k = 0; k < NI; ++k) off[k] = 0;
+        int64_t rem = row;
+#pragma unroll
+        for (int a = kMaxRank - 2; a >= 0; --a) {
+            if (a < m.outer.rank) {
+                const int64_t q = a ? rem / m.outer.ext[a] : 0, c = a ? rem - q * m.outer.ext[a] : rem;
+                rem = q;
+#pragma unroll
+                for (int k = 0; k < NI; ++k)
+                    if (k < ops.n) off[k] += c * ops.o[k].st[a];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < NI; ++k) {
+            if (k >= ops.n || (!first && ((m.column >> k) & 1u))) continue;
+            const T *p = static_cast<const T *>(ops.o[k].p) + off[k];
+            T *e = reinterpret_cast<T *>(&in[k]);
+            if ((m.splat >> k) & 1u) {
+                const T b = p[0];
+#pragma unroll
+                for (int j = 0; j < V; ++j) e[j] = b;
+            } else if (full) {
+                in[k] = (m.column >> k) & 1u ? load_any16<false>(p + c0) : load_any16<true>(p + c0);
+            } else {
+#pragma unroll
+                for (int j = 0; j < V; ++j) e[j] = c0 + j < m.last ? p[c0 + j] : T(0);
+            }
+        }
+    };
+    load(g, true);
+    uint32_t run = ~0u;
+    bool first = true;
+    for (int64_t row = g; row < m.rows; row += m.groups) {
+#pragma unroll
+        for (int k = 0; k < NI; ++k)
+            if (k < ops.n && (first || !((m.column >> k) & 1u))) slots[k * 256 + threadIdx.x] = in[k];
+        if (row + m.groups < m.rows) load(row + m.groups, false);
+        T r[V];
+        run_chain_vec<T, V>(ch, slots, ops.n, threadIdx.x, r, run);
+        run = ~m.step_column;
+        first = false;
+        T *o = out + row * m.last + c0;
+        if (full) {
+            Q rq;
+#pragma unroll
+            for (int j = 0; j < V; ++j) reinterpret_cast<T *>(&rq)[j] = r[j];
+            store_any16(o, rq);
+        } else {
+#pragma unroll
+            for (int j = 0; j < V; ++j)
+                if (c0 + j < m.last) o[j] = r[j];
+        }
+    }
+}
+
 // ---------------------------------------------------------------- unary maps
 // Contiguous n-element maps with 16-byte vectors; the scalar tail is the
 // last n % V elements.
@@ -659,6 +750,47 @@ int32_t launch_flat(const ChainDev &ch, FlatGroups &fg, hipStream_t strm) {
     return CHELIS_HIP_OK;
 }
 
+// The broadcast form: true when it takes the operands (see fused_rows_kernel)
+// and was launched; the general interpreter serves the rest (an operand
+// strided along the last axis, chains whose slots exceed 64 KiB of LDS, rows
+// shorter than a vector). The last step always runs per row: a chain of the
+// columns alone would leave nothing in r.
+template <typename T>
+bool launch_rows_map(const ChainDev &ch, const Operands &ops, const Shape &sh, T *out, hipStream_t strm) {
+    constexpr int64_t V = 16 / sizeof(T);
+    const size_t lds = (size_t)(ops.n + ch.n_steps) * 256 * 16;
+    const int last = sh.rank - 1;
+    if (sh.rank < 2 || lds > 65536 || sh.ext[last] < V || sh.ext[last] > (int64_t(1) << 31)) return false;
+    RowMap m{};
+    m.last = sh.ext[last], m.rows = 1, m.nv = (uint32_t)((m.last + V - 1) / V);
+    m.outer.rank = last;
+    for (int a = 0; a < last; ++a) m.outer.ext[a] = sh.ext[a], m.rows *= sh.ext[a];
+    for (int k = 0; k < ops.n; ++k) {
+        if (ops.o[k].st[last] != 0 && ops.o[k].st[last] != 1) return false;
+        if (ops.o[k].st[last] == 0) m.splat |= 1u << k;
+        bool column = true;
+        for (int a = 0; a < last; ++a) column = column && ops.o[k].st[a] == 0;
+        if (column) m.column |= 1u << k;
+    }
+    for (int s = 0; s + 1 < ch.n_steps; ++s) {
+        auto of_column = [&](int a) { return a >= 0 ? (m.column >> a) & 1u : (m.step_column >> (-a - 1)) & 1u; };
+        // a one-operand step leaves its second argument at input 0
+        const bool one = ch.op[s] >= CHELIS_FUSED_NEG && ch.op[s] <= CHELIS_FUSED_RELU;
+        if (ch.op[s] == CHELIS_FUSED_CONST || (of_column(ch.a0[s]) && (one || of_column(ch.a1[s]))))
+            m.step_column |= 1u << s;
+    }
+    // several rows per thread only where that saves loads or steps and the
+    // chip stays full: 8 waves per SIMD of 256 CUs and more
+    m.R = 1;
+    if (m.column)
+        while (m.R < 8 && m.rows * m.nv / (2 * m.R) >= int64_t(2048) * device_cus()) m.R *= 2;
+    m.groups = (m.rows + m.R - 1) / m.R;
+    const int64_t blocks = (m.groups * m.nv + 255) / 256;
+    if (!grid_fits(blocks, 256)) return false;
+    fused_rows_kernel<T><<<(unsigned)blocks, 256, lds, strm>>>(ch, ops, m, out);
+    return true;
+}
+
 void add_group(FlatGroups &fg, const chelis_gpu_tensor *const *inputs, int32_t n_inputs, const chelis_gpu_tensor *out,
                const int64_t (*st)[kMaxRank]) {
     FlatGroup &g = fg.g[fg.n++];
@@ -759,6 +891,11 @@ extern "C" int32_t chelis_hip_fused_elementwise(const chelis_fused_chain *chain,
     for (int32_t k = 0; k < n_inputs; ++k) {
         ops.o[k].p = inputs[k]->data;
         for (int a = 0; a < kMaxRank; ++a) ops.o[k].st[a] = st[k][a];
+    }
+    if (out->dtype == CHELIS_DTYPE_F32 ? launch_rows_map<float>(ch, ops, sh, (float *)out->data, strm)
+                                       : launch_rows_map<double>(ch, ops, sh, (double *)out->data, strm)) {
+        CHELIS_LAUNCH_CHECK();
+        return CHELIS_HIP_OK;
     }
     int64_t blocks = (out->count + 255) / 256;
     if (blocks > 8192) blocks = 8192;

@@ -402,6 +402,93 @@ __global__ __launch_bounds__(256) void reduce_cols4_kernel(ChainDev ch, LeafSrc 
     }
 }
 
+// Columns with a chain leaf over at most kChainPreloadInputs inputs: the
+// vector interpreter on four leaves of a column at a time (one op dispatch,
+// one LDS access per slot for the four), the next four leaves' loads in
+// flight meanwhile. A workgroup covers jw columns (a power of two up to 64)
+// and 256 / jw adjacent groups of 32 leaves, whose totals join in LDS in
+// order: one total per column of an aligned run of 8192 / jw leaves. An
+// input that does not move along the reduced axis is loaded once.
+// ([16384,4096] f32, sum (x - mean[col])^2 over the rows: 469 us one leaf per
+// interpreter run with the leaves in scratch memory.)
+template <typename T, Rk K, int NIN>
+__global__ __launch_bounds__(256) void reduce_cols_chain_kernel(ChainDev ch, LeafSrc src, int64_t n, int64_t inner,
+                                                                int64_t groups, int jshift, T *__restrict__ out_v,
+                                                                bool last) {
+    constexpr int G = 32, V = 4, NB = G / V;
+    struct alignas(16) Q {
+        T v[V];
+    };
+    extern __shared__ __align__(16) unsigned char cols_lds[];
+    Q *slots = reinterpret_cast<Q *>(cols_lds);
+    __shared__ T tot[NB][256];
+    const int tid = threadIdx.x, jw = 1 << jshift, gw = 256 >> jshift;
+    const int64_t jblocks = (inner + jw - 1) >> jshift;
+    int64_t b = blockIdx.x;
+    const int64_t jb = b % jblocks;
+    b /= jblocks;
+    const int64_t gb = b % groups, o = b / groups;
+    const int64_t jt = (jb << jshift) + (tid & (jw - 1)), j = jt < inner ? jt : inner - 1;
+    const int64_t i0 = (gb * gw + (tid >> jshift)) * G;
+    const T *p[NIN];
+#pragma unroll
+    for (int k = 0; k < NIN; ++k) p[k] = static_cast<const T *>(src.p[k]) + o * src.so[k] + j * src.si[k];
+    Q in[NIN];
+    auto load = [&](int t) {
+#pragma unroll
+        for (int k = 0; k < NIN; ++k) {
+            if (src.sn[k] == 0) {
+                if (t == 0) {
+                    const T x = *p[k];
+#pragma unroll
+                    for (int e = 0; e < V; ++e) in[k].v[e] = x;
+                }
+            } else {
+                // a leaf past the end reads the last one; it is not used
+#pragma unroll
+                for (int e = 0; e < V; ++e) {
+                    const int64_t i = i0 + t * V + e;
+                    in[k].v[e] = __builtin_nontemporal_load(p[k] + (i < n ? i : n - 1) * src.sn[k]);
+                }
+            }
+        }
+    };
+    load(0);
+#pragma unroll 1
+    for (int t = 0; t < NB; ++t) {
+#pragma unroll
+        for (int k = 0; k < NIN; ++k) slots[k * 256 + tid] = in[k];
+        if (t + 1 < NB) load(t + 1);
+        T r[V];
+        int64_t ri[V] = {0, 0, 0, 0};
+        run_chain_vec<T, V>(ch, slots, NIN, tid, r);
+#pragma unroll
+        for (int e = 0; e < V; ++e)
+            if (i0 + t * V + e >= n) r[e] = identity<T, K>();
+        ordered_tree<T, K, V>(r, ri);
+        tot[t][tid] = r[0];
+    }
+    T v[NB];
+    int64_t vi[NB] = {};
+#pragma unroll
+    for (int t = 0; t < NB; ++t) v[t] = tot[t][tid];
+    ordered_tree<T, K, NB>(v, vi);
+    // the groups of a column, in order, one level at a time
+    T a = v[0];
+    int64_t ia = 0;
+    for (int w = gw; w > 1; w >>= 1) {
+        __syncthreads();
+        tot[0][tid] = a;
+        __syncthreads();
+        if ((tid >> jshift) < w / 2) {
+            const int at = ((tid >> jshift) << (jshift + 1)) + (tid & (jw - 1));
+            a = tot[0][at];
+            combine<T, K>(a, ia, tot[0][at + jw], 0);
+        }
+    }
+    if (tid < jw && jt < inner) out_v[(o * groups + gb) * inner + jt] = last ? finalize<T, K>(a) : a;
+}
+
 template <typename T>
 __global__ void fill_kernel(T *p, int64_t n, T v) {
     const int64_t i = (int64_t)blockIdx.x * kReduceThreads + threadIdx.x;
@@ -527,6 +614,7 @@ struct Pass {
     bool vec;       // contiguous rows with 16-byte loads
     int S;          // rows: segments per wave
     bool cols4;     // columns: four waves per 128-leaf group
+    int jshift;     // columns, chain leaves: log2 of the columns per workgroup (reduce_cols_chain_kernel), or -1
     int64_t n;      // leaves per output this pass
     int64_t groups; // partials per output it writes
     int join = 0;   // rows, chain leaves: 2 or 4 groups joined in the workgroup, the pass writing the result
@@ -537,6 +625,8 @@ constexpr int kMaxPasses = 16;
 // before the interpreter runs.
 constexpr int kChainPreloadInputs = 3;
 constexpr int kChainSegments = 4;
+// Dynamic LDS of the column form, beside its 8 or 16 KiB of totals.
+constexpr size_t kColsChainLds = 40960;
 
 // The pass sequence: partials of pass i are the leaves of pass i + 1 and
 // live in a buffer 256-byte aligned, so their row alignment depends only
@@ -581,9 +671,19 @@ int plan_passes(const ChainDev &ch, bool chain, const LeafSrc &src, int64_t oute
         }
         // columns: 128-leaf groups per block when 64 columns fill a wave
         const bool cols4 = !rows && inner >= 64 && grid_fits(outer * ((cur_n + 127) / 128) * ((inner + 63) / 64), 256);
-        const int64_t G = rows ? unit * S : (cols4 ? 128 : 32);
+        // columns with a chain leaf: the vector interpreter where its slots fit
+        int jshift = -1;
+        if (!rows && use_chain && !has_index(K) && n_in <= kChainPreloadInputs &&
+            (size_t)(n_in + ch.n_steps) * 256 * 4 * sizeof(T) <= kColsChainLds) {
+            jshift = 0;
+            while (jshift < 6 && (int64_t(1) << jshift) < inner) ++jshift;
+            const int64_t leaves = 8192 >> jshift;
+            if (!grid_fits(outer * ((cur_n + leaves - 1) / leaves) * ((inner + (1 << jshift) - 1) >> jshift), 256))
+                jshift = -1;
+        }
+        const int64_t G = rows ? unit * S : (jshift >= 0 ? 8192 >> jshift : (cols4 ? 128 : 32));
         const int64_t groups = (cur_n + G - 1) / G;
-        passes[i] = Pass{vec, S, cols4, cur_n, groups};
+        passes[i] = Pass{vec, S, cols4, jshift, cur_n, groups};
         if (groups == 1) return i + 1;
         // a contiguous chain leaf over 2 or 4 groups per row, rows filling
         // whole workgroups: the workgroup joins each row's groups itself
@@ -741,6 +841,18 @@ int32_t run_reduce(const ChainDev &ch, bool chain, LeafSrc src, int64_t outer, i
             }
 #undef CHELIS_ROWS_CASE
 #undef CHELIS_ROWS_LAUNCH
+        } else if (ps.jshift >= 0) {
+            if constexpr (kChainable<K>) {
+                const int64_t jblocks = (inner + (1 << ps.jshift) - 1) >> ps.jshift;
+                const unsigned grid = (unsigned)(outer * groups * jblocks);
+                const size_t lds = (size_t)(s.n_in + ch.n_steps) * 256 * 4 * sizeof(T);
+                if (s.n_in == 1)
+                    reduce_cols_chain_kernel<T, K, 1><<<grid, 256, lds, st>>>(ch, s, cur_n, inner, groups, ps.jshift, dst_v, last);
+                else if (s.n_in == 2)
+                    reduce_cols_chain_kernel<T, K, 2><<<grid, 256, lds, st>>>(ch, s, cur_n, inner, groups, ps.jshift, dst_v, last);
+                else
+                    reduce_cols_chain_kernel<T, K, 3><<<grid, 256, lds, st>>>(ch, s, cur_n, inner, groups, ps.jshift, dst_v, last);
+            }
         } else if (cols4) {
             const unsigned grid = (unsigned)(outer * groups * ((inner + 63) / 64));
             bool done = false;

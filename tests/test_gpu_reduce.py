@@ -322,3 +322,20 @@ def test_column_sum_of_a_strided_view():
     d = C.to_device(big)
     view = d.view((1024, 1024), (1031, 1))
     assert bits_equal(C.reduce("sum", view, 0).numpy(), O.sum_axis(np.ascontiguousarray(big[:, :1024]), 0))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n,inner", [(1, 3), (31, 64), (33, 5), (128, 64), (129, 65), (1025, 8), (8193, 1 + 1), (700, 200)])
+def test_column_chain_leaves_on_the_vector_interpreter(dtype, n, inner):
+    """sum and max over the rows of (x - mean[col])^2 at the edges of the
+    leaf groups and column runs, the mean's stride 0 along the reduced axis:
+    the tree over numpy's leaves bit for bit."""
+    rng = np.random.default_rng(n + inner)
+    x = rng.standard_normal((2, n, inner)).astype(dtype)
+    mean = rng.standard_normal(inner).astype(dtype)
+    dx, dm = C.to_device(x), C.to_device(mean).view((2, n, inner), (0, 0, 1))
+    ch = C.fused_chain([("sub", 0, 1), ("mul", ("s", 0), ("s", 0))])
+    leaves = (x - mean) * (x - mean)
+    got = C.reduce("sum", [dx, dm], 1, chain=ch).numpy()
+    assert np.array_equal(got, O.sum_axis(leaves, 1))
+    assert np.array_equal(C.reduce("max", [dx, dm], 1, chain=ch).numpy(), leaves.max(1))

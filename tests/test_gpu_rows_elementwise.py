@@ -705,3 +705,33 @@ def test_causal_attention_fused_against_the_oracle(B, H, S):
     assert np.abs(o - ref).max() <= 1e-5 * np.abs(ref).max()
     big = np.abs(ref) >= np.sqrt(np.mean(ref ** 2))
     assert np.all(np.abs(o - ref)[big] <= 1e-5 * np.abs(ref)[big])
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("shape", [(5, 4), (7, 33), (300, 1000), (3, 65, 130), (4100, 1031)])
+def test_fused_chain_broadcast_forms(dtype, shape):
+    """Operands per column, per row, per element and one for all against a
+    tensor, rows of whole and partial vectors, a start off a 16-byte boundary
+    and (the largest) several rows per thread: the numpy chain's bits."""
+    rng = np.random.default_rng(sum(shape))
+    n = shape[-1]
+    size = int(np.prod(shape))
+    flat = rng.standard_normal(size + 1).astype(dtype)
+    x = flat[1:].reshape(shape)
+    col, var = rng.standard_normal(n).astype(dtype), rng.random(n).astype(dtype)
+    row = rng.standard_normal(shape[:-1]).astype(dtype)
+    tight = [int(np.prod(shape[a + 1:])) for a in range(len(shape))]
+    rowst = [t // n for t in tight[:-1]] + [0]
+    dx = C.to_device(flat).view(shape, tight, 1)
+    dcol, dvar = (C.to_device(a).view(shape, [0] * (len(shape) - 1) + [1]) for a in (col, var))
+    drow = C.to_device(row).view(shape, rowst)
+    done = C.to_device(np.array([1.5], dtype)).view(shape, [0] * len(shape))
+    out = C.empty(shape, dtype)
+    ch = C.fused_chain([("const", 0, 0, 1e-5), ("add", 2, ("s", 0)), ("sqrt", ("s", 1)), ("sub", 0, 1),
+                        ("div", ("s", 3), ("s", 2)), ("mul", ("s", 4), 3), ("add", ("s", 5), 4)])
+    C.fused_elementwise(ch, [dx, dcol, dvar, drow, done], out)
+    want = (x - col) / np.sqrt(var + dtype(1e-5)) * row[..., None] + dtype(1.5)
+    assert bits_equal(out.numpy(), want.astype(dtype)), mismatch_report(out.numpy(), want.astype(dtype))
+    # a chain of the columns alone
+    C.fused_elementwise(C.fused_chain([("add", 0, 1)]), [dcol, dvar], out)
+    assert bits_equal(out.numpy(), np.broadcast_to(col + var, shape).astype(dtype))
