@@ -490,6 +490,44 @@ __global__ __launch_bounds__(256) void gather_kernel(const U *__restrict__ value
     }
 }
 
+// Dense rows of whole dwords, at least one 16-byte vector each: a thread
+// copies one vector of a row (any dword boundary; the row's last vector is
+// the one that ends it, so it may repeat a part of the one before). The
+// failing index is keyed by its row's first element, the lowest.
+// (8192 rows of 2 KiB from a [50000, 512] table: 24.6 us one element per
+// thread, with three divisions each.)
+typedef uint32_t U4 __attribute__((ext_vector_type(4), aligned(4)));
+template <typename I>
+__global__ __launch_bounds__(256) void gather_rows_kernel(const uint32_t *__restrict__ values,
+                                                          const I *__restrict__ idx, View8 iv,
+                                                          uint32_t *__restrict__ out, GatherGeom g, int64_t words,
+                                                          uint32_t nv, int64_t items, uint64_t seq,
+                                                          unsigned long long *rec) {
+    const int64_t id = (int64_t)blockIdx.x * kSelectThreads + threadIdx.x;
+    unsigned long long k = 0ull;
+    if (id < items) {
+        const int64_t t = id / nv;
+        const int64_t at = (id - t * nv) * 4, w = at + 4 <= words ? at : words - 4;
+        const int64_t j = t % g.index_count, b = t / g.index_count;
+        const int64_t x = (int64_t)idx[logical_offset(iv, (b / g.outer_per_batch) * g.index_count + j)];
+        U4 v = {0, 0, 0, 0};
+        if (x < 0 || x >= g.axis_size) k = fail_key(seq, t * g.after, kDomain);
+        else v = *reinterpret_cast<const U4 *>(values + (b * g.axis_size + x) * words + w);
+        __builtin_nontemporal_store(v, reinterpret_cast<U4 *>(out + t * words + w));
+    }
+    merge_failures(k, rec);
+}
+
+// A dense copy, one 16-byte vector per thread (the last ends the array).
+__global__ __launch_bounds__(256) void copy_words_kernel(const uint32_t *__restrict__ x, uint32_t *__restrict__ y,
+                                                         int64_t words) {
+    const int64_t at = ((int64_t)blockIdx.x * kSelectThreads + threadIdx.x) * 4;
+    if (at >= words) return;
+    const int64_t w = at + 4 <= words ? at : words - 4;
+    __builtin_nontemporal_store(__builtin_nontemporal_load(reinterpret_cast<const U4 *>(x + w)),
+                                reinterpret_cast<U4 *>(y + w));
+}
+
 // ---------------------------------------------------------------- ordered scan
 // [05-OP-33] cumsum (kernels.rs:2793 ordered_scan, with the C lane's
 // accumulation, crates/chelis-runtime/src/lib.rs:7020-7105): one thread per
@@ -595,6 +633,7 @@ __global__ __launch_bounds__(256) void pad_kernel(const U *__restrict__ x, U *__
 // (crates/chelis-backend-hip/src/kernels.rs:2599-2765).
 struct ScatterGeom {
     int64_t axis_size, after, index_count, outer_per_batch, total;  // hyperplane form
+    int64_t span;                                                  // elements per position: 1, or a row's
     int32_t elements, rank, axis;                                  // ScatterElements
     int64_t idx_shape[8], target_shape[8];
 };
@@ -631,7 +670,7 @@ __global__ __launch_bounds__(256) void scatter_keys_kernel(const I *__restrict__
             }
             keys[i] = ok ? (K)dst : sentinel;
             pos[i] = (K)i;
-            if (!ok) k = fail_key(seq, i, kDomain);
+            if (!ok) k = fail_key(seq, i * g.span, kDomain);
         }
         merge_failures(k, rec);
     }
@@ -726,6 +765,178 @@ __global__ __launch_bounds__(256) void scatter_add_kernel(const K *__restrict__ 
         }
         if constexpr (!Dt<DT>::kFloat) merge_failures(k, rec);
     }
+}
+
+// ---- whole rows (the axes after the scattered one hold at least a quarter
+// of a wave's columns): one key per row of updates instead of one per
+// element is sorted, and a run is applied by waves with a column per lane.
+// (8192 updates of 512 columns into [50000, 512], word-like ids: the sort of
+// 4.2 million pairs took 210 us and the fold of the runs, one lane each with
+// its carry stack in scratch memory, 405.)
+
+// The last update of each destination row's run, copied.
+template <typename U, typename K>
+__global__ __launch_bounds__(256) void scatter_last_rows_kernel(const K *__restrict__ skeys,
+                                                                const K *__restrict__ spos, int64_t m, K sentinel,
+                                                                const U *__restrict__ upd, View8 uv, int64_t after,
+                                                                int64_t chunks, U *__restrict__ out) {
+    const int64_t item = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t p = item / chunks, c = (item - p * chunks) * 64 + (threadIdx.x & 63);
+    if (p >= m || c >= after) return;
+    const K d = skeys[p];
+    if (d == sentinel || (p + 1 < m && skeys[p + 1] == d)) return;
+    out[(int64_t)d * after + c] = upd[logical_offset(uv, (int64_t)spos[p] * after + c)];
+}
+
+// The pair tree over N leaves, leaf 0 the target's value and leaf i the
+// run's update i - 1; past `len` updates the exact identity (-0, or 0).
+template <int DT>
+__device__ inline typename AddNode<DT>::A add_identity() {
+    if constexpr (Dt<DT>::kFloat) return (typename AddNode<DT>::A)(-0.0);
+    else return 0;
+}
+template <int DT, int N>
+__device__ inline bool tree_join(typename AddNode<DT>::A (&v)[N]) {
+    bool ok = true;
+#pragma unroll
+    for (int w = N; w > 1; w >>= 1)
+#pragma unroll
+        for (int i = 0; i < w / 2; ++i) ok = AddNode<DT>::add(v[2 * i], v[2 * i + 1], &v[i]) && ok;
+    return ok;
+}
+
+constexpr int kLongRun = 32;  // updates: such runs go to scatter_add_long_kernel
+
+// A wave per (sorted position, 64 columns); the run's first position folds
+// it. Every update's load is issued before the first add.
+template <int DT, typename K>
+__global__ __launch_bounds__(256) void scatter_add_rows_kernel(const K *__restrict__ skeys,
+                                                               const K *__restrict__ spos, int64_t m, K sentinel,
+                                                               const typename Dt<DT>::S *__restrict__ upd, View8 uv,
+                                                               int64_t after, int64_t chunks, int64_t total,
+                                                               typename Dt<DT>::S *__restrict__ out, uint64_t seq,
+                                                               unsigned long long *rec) {
+    using N = AddNode<DT>;
+    using A = typename N::A;
+    const int lane = threadIdx.x & 63;
+    const int64_t item = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t p = item / chunks;
+    if (p >= m) return;
+    const K d = skeys[p];
+    if (d == sentinel || (p > 0 && skeys[p - 1] == d)) return;
+    const uint64_t same = __ballot(p + lane < m && skeys[p + lane < m ? p + lane : p] == d);
+    const int len = ~same ? __builtin_ctzll(~same) : 64;
+    if (len >= kLongRun) return;
+    const int64_t col = (item - p * chunks) * 64 + lane;
+    const bool live = col < after;
+    const int64_t c = live ? col : after - 1, dst = (int64_t)d * after + c;
+    auto fold = [&](auto size) {
+        constexpr int L = decltype(size)::value;
+        A v[L];
+        v[0] = N::leaf(out[dst]);
+#pragma unroll
+        for (int i = 1; i < L; ++i) {
+            const int64_t q = (int64_t)spos[p + (i <= len ? i : len) - 1];
+            v[i] = N::leaf(upd[logical_offset(uv, q * after + c)]);
+        }
+#pragma unroll
+        for (int i = 1; i < L; ++i) v[i] = i <= len ? v[i] : add_identity<DT>();
+        const bool ok = tree_join<DT, L>(v);
+        unsigned long long k = 0ull;
+        if (ok && live) out[dst] = N::store(v[0]);
+        if (!ok && live) k = fail_key(seq, total + dst, kOverflow);
+        if constexpr (!Dt<DT>::kFloat) merge_failures(k, rec);
+    };
+    if (len < 2) fold(std::integral_constant<int, 2>{});
+    else if (len < 4) fold(std::integral_constant<int, 4>{});
+    else if (len < 8) fold(std::integral_constant<int, 8>{});
+    else if (len < 16) fold(std::integral_constant<int, 16>{});
+    else fold(std::integral_constant<int, 32>{});
+}
+
+// Runs of at least kLongRun updates: a workgroup per (16 sorted positions,
+// 64 columns) whose first position lies in a run that began in the 16
+// before it (every such run has exactly one). Each step folds 128 leaves, 32
+// per wave in registers with all loads in flight, joined through LDS, and
+// pushes the total on a carry stack of aligned 128-leaf subtrees.
+template <int DT, typename K>
+__global__ __launch_bounds__(256) void scatter_add_long_kernel(const K *__restrict__ skeys,
+                                                               const K *__restrict__ spos, int64_t m, K sentinel,
+                                                               const typename Dt<DT>::S *__restrict__ upd, View8 uv,
+                                                               int64_t after, int64_t chunks, int64_t total,
+                                                               typename Dt<DT>::S *__restrict__ out, uint64_t seq,
+                                                               unsigned long long *rec) {
+    using N = AddNode<DT>;
+    using A = typename N::A;
+    constexpr int L = 32, STEP = 4 * L, LEVELS = 25;  // 2^31 updates are 2^24 steps
+    static_assert(L == kLongRun, "the first step's first wave is full");
+    __shared__ A tot[4][64], stack[LEVELS][64];
+    __shared__ int held[4], good[4][64];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t p16 = (int64_t)blockIdx.x / chunks * 16;
+    const K d = skeys[p16];
+    if (d == sentinel || p16 + 16 >= m || skeys[p16 + 16] != d) return;
+    const int back = p16 > 0 ? 16 : 0;
+    const bool mine = lane >= 1 && lane <= back && skeys[p16 - (lane <= back ? lane : 0)] == d;
+    const int before = __popcll(__ballot(mine));
+    if (before == 16) return;  // an earlier workgroup's run
+    const int64_t s = p16 - before;
+    if (s + kLongRun > m || skeys[s + kLongRun - 1] != d) return;
+    const int64_t col = (int64_t)(blockIdx.x % chunks) * 64 + lane;
+    const bool live = col < after;
+    const int64_t c = live ? col : after - 1, dst = (int64_t)d * after + c;
+    bool ok = true;
+    uint64_t cnt = 0;
+    for (int64_t leaf0 = 0;; leaf0 += STEP) {
+        // leaf 0 is the target, leaf q the update at sorted position s + q - 1
+        const int64_t q = leaf0 + w * L + (lane & 31);
+        const int64_t at = s + (q > 0 ? q - 1 : 0);
+        const bool in_run = at < m && skeys[at < m ? at : s] == d;
+        const uint32_t mask = (uint32_t)__ballot(in_run);
+        const int64_t row = (int64_t)spos[in_run ? at : s];
+        const uint32_t row_lo = (uint32_t)row, row_hi = (uint32_t)(row >> 32);
+        A v[L];
+#pragma unroll
+        for (int i = 0; i < L; ++i) {
+            const int64_t r = (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)row_hi, i) << 32 |
+                                        (uint32_t)__builtin_amdgcn_readlane((int)row_lo, i));
+            v[i] = N::leaf(upd[logical_offset(uv, r * after + c)]);
+        }
+        if (leaf0 == 0 && w == 0) v[0] = N::leaf(out[dst]);
+#pragma unroll
+        for (int i = 0; i < L; ++i) v[i] = (mask >> i) & 1u ? v[i] : add_identity<DT>();
+        ok = tree_join<DT, L>(v) && ok;
+        tot[w][lane] = v[0];
+        if (lane == 0) held[w] = mask == ~0u;
+        __syncthreads();
+        const bool more = held[0] && held[1] && held[2] && held[3];
+        if (w == 0) {
+            A u[4] = {tot[0][lane], tot[1][lane], tot[2][lane], tot[3][lane]};
+            ok = tree_join<DT, 4>(u) && ok;
+            int lv = 0;
+            for (uint64_t b = cnt; b & 1; b >>= 1, ++lv) ok = N::add(stack[lv][lane], u[0], &u[0]) && ok;
+            stack[lv][lane] = u[0];
+            ++cnt;
+        }
+        __syncthreads();
+        if (!more) break;
+    }
+    good[w][lane] = ok;
+    __syncthreads();
+    if (w != 0) return;
+    ok = good[0][lane] && good[1][lane] && good[2][lane] && good[3][lane];
+    A acc{};
+    bool have = false;
+    for (int lv = 0; (cnt >> lv) != 0; ++lv)
+        if ((cnt >> lv) & 1) {
+            if (have) ok = N::add(stack[lv][lane], acc, &acc) && ok;
+            else acc = stack[lv][lane];
+            have = true;
+        }
+    unsigned long long k = 0ull;
+    if (ok && live) out[dst] = N::store(acc);
+    if (!ok && live) k = fail_key(seq, total + dst, kOverflow);
+    if constexpr (!Dt<DT>::kFloat) merge_failures(k, rec);
 }
 
 // ---------------------------------------------------------------- host: the failure channel
@@ -977,6 +1188,24 @@ int32_t launch_gather(const chelis_gpu_tensor *values, const chelis_gpu_tensor *
     hipStream_t st = stream();
     if (!st) return set_error(CHELIS_HIP_EHIP, "no HIP device");
     if (!g.total) return CHELIS_HIP_OK;
+    const int64_t words = g.after * (int64_t)sizeof(U) / 4, nv = (words + 3) / 4, items = g.total / g.after * nv;
+    auto dwords = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 3) == 0; };
+    if (is_contiguous(values) && (g.after * (int64_t)sizeof(U)) % 4 == 0 && words >= 4 && nv <= 0x7fffffff &&
+        dwords(values->data) && dwords(out->data) && grid_fits((items + 255) / 256, 256)) {
+        const unsigned grid = (unsigned)((items + 255) / 256);
+        const uint32_t *v = static_cast<const uint32_t *>(values->data);
+        uint32_t *o = static_cast<uint32_t *>(out->data);
+        if (indices->dtype == CHELIS_DTYPE_I32)
+            gather_rows_kernel<int32_t><<<grid, 256, 0, st>>>(v, static_cast<const int32_t *>(indices->data),
+                                                             view_of(indices), o, g, words, (uint32_t)nv, items, s.seq,
+                                                             s.rec);
+        else
+            gather_rows_kernel<int64_t><<<grid, 256, 0, st>>>(v, static_cast<const int64_t *>(indices->data),
+                                                             view_of(indices), o, g, words, (uint32_t)nv, items, s.seq,
+                                                             s.rec);
+        CHELIS_LAUNCH_CHECK();
+        return CHELIS_HIP_OK;
+    }
     const unsigned blocks = (unsigned)map_blocks(g.total);
     if (indices->dtype == CHELIS_DTYPE_I32)
         gather_kernel<U, int32_t><<<dim3(blocks), dim3(256), 0, st>>>(
@@ -1278,6 +1507,26 @@ extern "C" int32_t chelis_hip_pad(const chelis_gpu_tensor *x, const int64_t *lo,
 }
 
 namespace {
+// Rows of at least 16 columns take the row kernels; narrower ones (and
+// ScatterElements) a lane per element.
+bool scatter_by_rows(int32_t mode, const ScatterGeom &g) { return mode != 2 && g.after >= 16; }
+
+// out = target: nothing when they are one tensor, a dense copy where both
+// are contiguous whole dwords, else the strided copy of pad.
+int32_t copy_target(const chelis_gpu_tensor *target, const chelis_gpu_tensor *out, hipStream_t st) {
+    const int64_t zeros[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    const int64_t bytes = out->count * dtype_width(out->dtype), blocks = (bytes + 4095) / 4096;
+    auto dwords = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 3) == 0; };
+    if (!is_contiguous(target) || bytes % 4 || bytes < 16 || !dwords(target->data) || !dwords(out->data) ||
+        !grid_fits(blocks, 256))
+        return chelis_hip_pad(target, zeros, 0, out);
+    if (target->data == out->data) return CHELIS_HIP_OK;
+    copy_words_kernel<<<(unsigned)blocks, 256, 0, st>>>(static_cast<const uint32_t *>(target->data),
+                                                       static_cast<uint32_t *>(out->data), bytes / 4);
+    CHELIS_LAUNCH_CHECK();
+    return CHELIS_HIP_OK;
+}
+
 // The scatter's passes over keys of width K (destinations and positions):
 // the target copied into out, the keys, the stable sort, the runs applied.
 template <typename K>
@@ -1285,11 +1534,18 @@ int32_t run_scatter(int32_t mode, const chelis_gpu_tensor *target, const chelis_
                     const chelis_gpu_tensor *updates, const chelis_gpu_tensor *out, const ScatterGeom &g,
                     const Sink &s) {
     hipStream_t st = stream();
-    const int64_t zeros[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (int32_t r = chelis_hip_pad(target, zeros, 0, out)) return r;
-    const int64_t n = g.total;
+    if (int32_t r = copy_target(target, out, st)) return r;
+    // whole rows: a key per row of updates (destinations are rows)
+    const bool rows = scatter_by_rows(mode, g);
+    const int64_t after = rows ? g.after : 1, total = g.total, n = total / after;
     if (!n) return CHELIS_HIP_OK;
-    const K sentinel = (K)out->count;
+    const K sentinel = (K)(out->count / after);
+    ScatterGeom kg = g;
+    kg.span = after;
+    if (rows) kg.after = 1, kg.total = n;
+    const int64_t chunks = (after + 63) / 64;
+    if (rows && (!grid_fits((n * chunks + 3) / 4, 256) || !grid_fits((n + 15) / 16 * chunks, 256)))
+        return set_error(CHELIS_HIP_EUNSUPPORTED, "scatter: too many rows of updates");
     int end_bit = 1;
     while (end_bit < (int)(8 * sizeof(K)) && ((uint64_t)sentinel >> end_bit) != 0) ++end_bit;
     size_t temp = 0;
@@ -1305,17 +1561,56 @@ int32_t run_scatter(int32_t mode, const chelis_gpu_tensor *target, const chelis_
     const View8 iv = view_of(indices), uv = view_of(updates);
     const unsigned blocks = (unsigned)map_blocks(n);
     if (indices->dtype == CHELIS_DTYPE_I32)
-        scatter_keys_kernel<int32_t, K><<<blocks, 256, 0, st>>>(static_cast<const int32_t *>(indices->data), iv, g,
+        scatter_keys_kernel<int32_t, K><<<blocks, 256, 0, st>>>(static_cast<const int32_t *>(indices->data), iv, kg,
                                                                sentinel, keys, pos, s.seq, s.rec);
     else
-        scatter_keys_kernel<int64_t, K><<<blocks, 256, 0, st>>>(static_cast<const int64_t *>(indices->data), iv, g,
+        scatter_keys_kernel<int64_t, K><<<blocks, 256, 0, st>>>(static_cast<const int64_t *>(indices->data), iv, kg,
                                                                sentinel, keys, pos, s.seq, s.rec);
     if (hipGetLastError() != hipSuccess) rc = set_error(CHELIS_HIP_EHIP, "scatter: key launch failed");
     if (!rc && hipcub::DeviceRadixSort::SortPairs(tmp, temp, keys, skeys, pos, spos, (int)n, 0, end_bit, st) !=
                    hipSuccess)
         rc = set_error(CHELIS_HIP_EHIP, "scatter: the sort failed");
     if (!rc) {
-        if (mode != 1) {
+        if (rows) {
+            const unsigned items = (unsigned)((n * chunks + 3) / 4);
+            if (mode != 1) {
+#define CHELIS_SCATTER_LAST(U)                                                                                     \
+    scatter_last_rows_kernel<U, K><<<items, 256, 0, st>>>(skeys, spos, n, sentinel,                                \
+                                                          static_cast<const U *>(updates->data), uv, after, chunks, \
+                                                          static_cast<U *>(out->data))
+                switch (dtype_width(out->dtype)) {
+                    case 1: CHELIS_SCATTER_LAST(uint8_t); break;
+                    case 2: CHELIS_SCATTER_LAST(uint16_t); break;
+                    case 4: CHELIS_SCATTER_LAST(uint32_t); break;
+                    default: CHELIS_SCATTER_LAST(uint64_t);
+                }
+#undef CHELIS_SCATTER_LAST
+            } else {
+                const unsigned longs = (unsigned)((n + 15) / 16 * chunks);
+#define CHELIS_SCATTER_ADD_ROWS(DT)                                                                                \
+    case DT:                                                                                                       \
+        scatter_add_rows_kernel<DT, K><<<items, 256, 0, st>>>(                                                     \
+            skeys, spos, n, sentinel, static_cast<const typename Dt<DT>::S *>(updates->data), uv, after, chunks,   \
+            total, static_cast<typename Dt<DT>::S *>(out->data), s.seq, s.rec);                                    \
+        if (n >= kLongRun)                                                                                         \
+            scatter_add_long_kernel<DT, K><<<longs, 256, 0, st>>>(                                                 \
+                skeys, spos, n, sentinel, static_cast<const typename Dt<DT>::S *>(updates->data), uv, after,       \
+                chunks, total, static_cast<typename Dt<DT>::S *>(out->data), s.seq, s.rec);                        \
+        break;
+                switch (out->dtype) {
+                    CHELIS_SCATTER_ADD_ROWS(CHELIS_DTYPE_F32)
+                    CHELIS_SCATTER_ADD_ROWS(CHELIS_DTYPE_F64)
+                    CHELIS_SCATTER_ADD_ROWS(CHELIS_DTYPE_BF16)
+                    CHELIS_SCATTER_ADD_ROWS(CHELIS_DTYPE_F16)
+                    CHELIS_SCATTER_ADD_ROWS(CHELIS_DTYPE_I8)
+                    CHELIS_SCATTER_ADD_ROWS(CHELIS_DTYPE_I16)
+                    CHELIS_SCATTER_ADD_ROWS(CHELIS_DTYPE_I32)
+                    CHELIS_SCATTER_ADD_ROWS(CHELIS_DTYPE_I64)
+                    default: rc = set_error(CHELIS_HIP_EDOMAIN, "scatter: no add for this dtype");
+                }
+#undef CHELIS_SCATTER_ADD_ROWS
+            }
+        } else if (mode != 1) {
             switch (dtype_width(out->dtype)) {
                 case 1:
                     scatter_last_kernel<uint8_t, K><<<blocks, 256, 0, st>>>(
@@ -1373,7 +1668,8 @@ int32_t scatter_common(int32_t mode, const chelis_gpu_tensor *target, const chel
         return set_error(CHELIS_HIP_EUNSUPPORTED, "%s: more than 2^31 - 1 updates", names[mode]);
     Sink sink;
     if (int32_t r = open_sink(failure != nullptr, label, &sink, false, overflow)) return r;
-    const bool narrow = (uint64_t)out->count < 0xFFFFFFFFull && (uint64_t)g.total < 0xFFFFFFFFull;
+    const int64_t span = scatter_by_rows(mode, g) ? g.after : 1;
+    const bool narrow = (uint64_t)(out->count / span) < 0xFFFFFFFFull && (uint64_t)(g.total / span) < 0xFFFFFFFFull;
     const int32_t st = narrow ? run_scatter<uint32_t>(mode, target, indices, updates, out, g, sink)
                               : run_scatter<uint64_t>(mode, target, indices, updates, out, g, sink);
     if (st) return st;

@@ -494,3 +494,66 @@ def test_cumsum_of_a_broadcast_view():
     v = C.to_device(row).view((5, 3), (0, 1))
     out, f = C.cumsum(v, 0)
     assert f is None and out.numpy().tobytes() == O.cumsum("f32", np.broadcast_to(row, (5, 3)).copy(), 0)[0].tobytes()
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16", "i32", "i8"])
+@pytest.mark.parametrize("add", [False, True])
+@pytest.mark.parametrize("after", [16, 64, 65])
+def test_scatter_rows_at_the_run_edges(dt, add, after):
+    """Rows of one chunk of columns and of a partial second one, runs one
+    below, at and past the sizes the kernels change at (1, 2, 3, 31, 32, 33,
+    127, 128, 129, 300), placed so that runs start anywhere in a sixteen of
+    sorted positions, ids shuffled: the oracle's bits."""
+    rng = np.random.default_rng(after)
+    ids = np.repeat(np.arange(12) * 3, [1, 31, 2, 32, 3, 33, 15, 127, 128, 129, 5, 300])
+    ids = rng.permutation(ids).astype(np.int64)
+    if dt in ("f32", "bf16"):
+        t = rng.standard_normal((40, after)).astype(np.float32)
+        u = (rng.standard_normal((len(ids), after)) * 4).astype(np.float32)
+        if dt == "bf16":
+            t, u = O.narrow_encode("bf16", t), O.narrow_encode("bf16", u)
+    else:
+        t = rng.integers(-3, 4, (40, after)).astype(np.int32 if dt == "i32" else np.int8)
+        u = rng.integers(-1, 2, (len(ids), after)).astype(t.dtype)
+    want, first, _ = O.scatter(dt, t, ids, u, 0, add=add)
+    assert first == -1
+    out, failure = C.scatter(C.to_device(t), C.to_device(ids), C.to_device(u), 0, add=add)
+    assert failure is None and bits(out.numpy()).tobytes() == bits(want).tobytes()
+    # in place: the target is the result
+    d = C.to_device(t)
+    C.scatter(d, C.to_device(ids), C.to_device(u), 0, add=add, out=d)
+    assert bits(d.numpy()).tobytes() == bits(want).tobytes()
+
+
+@pytest.mark.parametrize("long", [False, True])
+def test_scatter_rows_failures_match_the_oracle(long):
+    """An index outside the axis fails at its row's first element, an i8 node
+    outside the width at its destination, short and long runs alike."""
+    ids = np.zeros(200 if long else 20, np.int64)
+    ids[: len(ids) // 2] = 3
+    t = np.full((5, 40), 100, np.int8)
+    u = np.ones((len(ids), 40), np.int8)
+    u[len(ids) // 2 :, 7] = 100
+    _, first, kind = O.scatter("i8", t, ids, u, 0, add=True)
+    assert first >= 0
+    _, failure = C.scatter(C.to_device(t), C.to_device(ids), C.to_device(u), 0, add=True)
+    assert failure[:2] == (first, kind)
+    ids[11] = 5
+    _, first, kind = O.scatter("i8", t, ids, u, 0, add=True)
+    _, failure = C.scatter(C.to_device(t), C.to_device(ids), C.to_device(u), 0, add=True)
+    assert failure[:2] == (first, kind)
+
+
+@pytest.mark.parametrize("dtype,after", [(np.float32, 4), (np.float32, 5), (np.float64, 2), (np.uint16, 8),
+                                         (np.uint16, 10), (np.int8, 16), (np.int8, 20), (np.int8, 18), (np.float32, 3)])
+def test_gather_rows_of_whole_and_partial_vectors(dtype, after):
+    rng = np.random.default_rng(after)
+    values = rng.integers(-100, 100, (2, 9, after)).astype(dtype)
+    idx = rng.integers(0, 9, (2, 37)).astype(np.int32)
+    want, first = O.gather(values, idx, 1, 1)[:2]
+    got, failure = C.gather(C.to_device(values), C.to_device(idx), 1, 1)
+    assert failure is None and got.numpy().tobytes() == want.tobytes()
+    idx[1, 5] = 9
+    want, first = O.gather(values, idx, 1, 1)[:2]
+    got, failure = C.gather(C.to_device(values), C.to_device(idx), 1, 1)
+    assert failure[0] == first and got.numpy().tobytes() == want.tobytes()
