@@ -454,3 +454,64 @@ def test_batched_projection_shape_with_per_batch_bias(act):
             ref = np.maximum(ref, 0.0)
         got = c[j][rows].astype(np.float64)
         assert np.abs(got - ref).max() / np.abs(ref).max() <= 1e-5, j
+
+
+def _binary32_bound(a, b):
+    """Any order of K binary32 products and sums: K + 2 roundings of 2^-24 of
+    sum |a b|, and the least subnormal per term."""
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    k = a.shape[-1]
+    return a64 @ b64, (k + 2) * 2.0 ** -24 * (np.abs(a64) @ np.abs(b64)) + k * 2.0 ** -149
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt", "strided"])
+@pytest.mark.parametrize("shape", [(16, 16, 33), (64, 64, 64), (65, 130, 100), (129, 257, 1000), (640, 2048, 96),
+                                   (1100, 3000, 161)])
+def test_binary32_pieces_at_the_tile_edges(shape, layout):
+    """Binary32 products on the bfloat16 cores (three pieces per value): whole
+    and partial tiles and K steps, 64- and 128-tiles, every staging layout,
+    rows off 16-byte boundaries; within the binary32 bound."""
+    M, N, K = shape
+    rng = np.random.default_rng(M + N + K)
+    a, b = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, N)).astype(np.float32)
+    if layout == "strided":
+        wa, wb = np.zeros((M, 3 * K), np.float32), np.zeros((K, 2 * N + 1), np.float32)
+        wa[:, ::3], wb[:, 1::2] = a, b
+        da = C.to_device(wa).view((M, K), (3 * K, 3))
+        db = C.to_device(wb).view((K, N), (2 * N + 1, 2), 1)
+    else:
+        da = C.to_device(a) if layout[0] == "n" else C.to_device(np.ascontiguousarray(a.T)).view((M, K), (1, M))
+        db = C.to_device(b) if layout[1] == "n" else C.to_device(np.ascontiguousarray(b.T)).view((K, N), (1, K))
+    c = C.matmul(da, db).numpy().astype(np.float64)
+    ref, bound = _binary32_bound(a, b)
+    assert (np.abs(c - ref) <= bound).all(), float((np.abs(c - ref) / bound).max())
+
+
+@pytest.mark.parametrize("sa,sb", [(1e-36, 1.0), (1e-42, 1e30), (1.0, 1e-40), (1e-20, 1e-22), (1e18, 1e18)])
+def test_binary32_pieces_at_the_ends_of_the_range(sa, sb):
+    """Operands whose pieces would fall below the normal numbers (computed by
+    the binary32 loop), sums among the subnormals, and sums near the top."""
+    rng = np.random.default_rng(3)
+    a = (rng.uniform(0.5, 1, (200, 160)) * sa).astype(np.float32)
+    b = (rng.uniform(-1, 1, (160, 136)) * sb).astype(np.float32)
+    a[:, 5] = 0.0
+    c = C.matmul(C.to_device(a), C.to_device(b)).numpy().astype(np.float64)
+    ref, bound = _binary32_bound(a, b)
+    assert (np.abs(c - ref) <= bound).all(), float((np.abs(c - ref) / bound).max())
+
+
+def test_binary32_pieces_infinities_nan_and_the_largest_values():
+    """An infinity or a NaN reaches the rows and columns it belongs to and no
+    other, a value that rounds past the largest bfloat16 stays exact, and sums
+    past the range are infinite: as the binary32 products give them."""
+    rng = np.random.default_rng(4)
+    a = rng.standard_normal((200, 64)).astype(np.float32)
+    b = rng.uniform(0.5, 1, (64, 200)).astype(np.float32)
+    a[3, 7], a[70, 9], a[130, 0] = np.inf, np.nan, np.float32(3.4028235e38)
+    a[131] = np.float32(3e38)
+    b[0, :] = 0.5
+    c = C.matmul(C.to_device(a), C.to_device(b)).numpy()
+    assert np.isposinf(c[3]).all() and np.isnan(c[70]).all() and np.isposinf(c[131]).all()
+    rest = np.delete(np.arange(200), [3, 70, 131])
+    ref, bound = _binary32_bound(a[rest], b)
+    assert (np.abs(c[rest] - ref) <= bound).all()
