@@ -391,6 +391,7 @@ __device__ inline void run_chain_vec(const ChainDev &ch, Q *slots, int n_in, int
             y[j] = reinterpret_cast<const T *>(&yq)[j];
         }
         apply_step_vec<T, V>(ch.op[st], x, y, ch.imm[st], r);
+        if (st + 1 == ch.n_steps) break;  // nothing reads the last step's slot
         Q rq;
 #pragma unroll
         for (int j = 0; j < V; ++j) reinterpret_cast<T *>(&rq)[j] = r[j];

@@ -277,9 +277,9 @@ struct RowMap {
     Shape outer;                 // the axes before the last
 };
 
-template <typename T>
+template <typename T, int NI>
 __global__ __launch_bounds__(256) void fused_rows_kernel(ChainDev ch, Operands ops, RowMap m, T *out) {
-    constexpr int V = 16 / sizeof(T), NI = CHELIS_FUSED_MAX_INPUTS;
+    constexpr int V = 16 / sizeof(T);
     using Q = typename Vec16F<T>::type;
     extern __shared__ __align__(16) unsigned char rows_lds[];
     Q *slots = reinterpret_cast<Q *>(rows_lds);
@@ -787,7 +787,9 @@ bool launch_rows_map(const ChainDev &ch, const Operands &ops, const Shape &sh, T
     m.groups = (m.rows + m.R - 1) / m.R;
     const int64_t blocks = (m.groups * m.nv + 255) / 256;
     if (!grid_fits(blocks, 256)) return false;
-    fused_rows_kernel<T><<<(unsigned)blocks, 256, lds, strm>>>(ch, ops, m, out);
+    // the operand count bounds the registers: three keep five waves per SIMD
+    if (ops.n <= 3) fused_rows_kernel<T, 3><<<(unsigned)blocks, 256, lds, strm>>>(ch, ops, m, out);
+    else fused_rows_kernel<T, CHELIS_FUSED_MAX_INPUTS><<<(unsigned)blocks, 256, lds, strm>>>(ch, ops, m, out);
     return true;
 }
 
