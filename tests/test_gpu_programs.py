@@ -227,3 +227,36 @@ def test_host_entry_count_mismatch_aborts():
             "C.host_entry('linreg_step', [np.zeros((4, 2)), np.zeros(2)], 2)")
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
     assert r.returncode != 0 and "linreg_step: expected 3 inputs, got 2" in r.stderr
+
+
+@pytest.mark.parametrize("B,S", [(1, 1), (2, 63), (1, 65), (3, 200)])
+def test_transformer_block_of_any_length(B, S):
+    """Sequences that are no multiple of the attention tile, shorter than one
+    and just past one: within 1e-5 relative of the oracle's block."""
+    D, F = 128, 256
+    rng = np.random.default_rng(S)
+    p = lambda *s: (rng.standard_normal(s) * 0.05).astype(np.float32)
+    one, zero = np.ones(D, np.float32), np.zeros(D, np.float32)
+    args = [rng.standard_normal((B, S, D)).astype(np.float32), one, zero, p(D, D), p(D), p(D, D), p(D), p(D, D), p(D),
+            p(D, D), p(D), one, zero, p(D, F), p(F), p(F, D), p(D)]
+    out = C.empty((B, S, D), np.float32)
+    C.program("transformer_block", [C.to_device(a) for a in args], [out])
+    x = args[0].astype(np.float64)
+    w = [a.astype(np.float64) for a in args[1:]]
+
+    def norm(v, g, b):
+        c = v - v.mean(-1, keepdims=True)
+        return c / np.sqrt((c * c).mean(-1, keepdims=True) + 1e-5) * g + b
+
+    h = norm(x, w[0], w[1])
+    q, k, v = ((h @ w[i] + w[i + 1]).reshape(B, S, D // 64, 64).transpose(0, 2, 1, 3) for i in (2, 4, 6))
+    s = q @ k.transpose(0, 1, 3, 2) / 8
+    s[..., np.triu(np.ones((S, S), bool), 1)] = -np.inf
+    e = np.exp(s - s.max(-1, keepdims=True))
+    o = ((e / e.sum(-1, keepdims=True)) @ v).transpose(0, 2, 1, 3).reshape(B, S, D)
+    x = x + o @ w[8] + w[9]
+    f = norm(x, w[10], w[11]) @ w[12] + w[13]
+    from math import erf
+    f = f * 0.5 * (1 + np.vectorize(erf)(f / np.sqrt(2.0)))
+    ref = x + f @ w[14] + w[15]
+    assert normwise(out.numpy(), ref) < 1e-5
