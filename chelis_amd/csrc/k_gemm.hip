@@ -366,11 +366,17 @@ __global__ __launch_bounds__(THREADS, (kMinWavesPerEu<T, TM>)) void gemm_mfma_ke
     const int64_t first = group * GM;
     const int64_t gsz = (tiles_m - first) < GM ? (tiles_m - first) : GM;
     const int64_t in_group = bid % (GM * tiles_n);
-    const int64_t m0 = (first + in_group % gsz) * BM;
-    const int64_t n0 = (in_group / gsz) * BN;
+    // this workgroup's rows and columns of C start at (mo, no); a last tile
+    // that would run past the end of an operand is moved back to end with it
+    // (m0, n0), so its loads are the interior tiles' and only the elements of
+    // its own it stores. Bounds checks on every load made such tiles the
+    // stragglers of the launch: 1000 x 3000 x 4000 with both operands stored
+    // along the outer axis, FIGSHIFT.
+    const int64_t mo = (first + in_group % gsz) * BM, no = (in_group / gsz) * BN;
+    const int64_t m0 = p.M >= BM && mo + BM > p.M ? p.M - BM : mo, n0 = p.N >= BN && no + BN > p.N ? p.N - BN : no;
     // causal 1: a tile wholly above the diagonal is never read (the whole
     // workgroup leaves before any barrier); causal 2: a[m][k] = 0 for k > m
-    if (p.causal == 1 && n0 > m0 + BM - 1) return;
+    if (p.causal == 1 && no > mo + BM - 1) return;
     int64_t K = (p.causal == 2 && m0 + BM < p.K) ? m0 + BM : p.K;
 
     const int64_t z = blockIdx.y;
@@ -400,7 +406,8 @@ __global__ __launch_bounds__(THREADS, (kMinWavesPerEu<T, TM>)) void gemm_mfma_ke
     Stage<T, BLAY, BN, BK, LD> sb0, sb1;
     const int64_t ksteps = (K + BK - 1) / BK;
     // an interior tile of aligned operands and whole K steps loads without checks
-    const bool inside = a_vec && b_vec && ALAY != 2 && BLAY != 2 && m0 + BM <= p.M && n0 + BN <= p.N && K % BK == 0;
+    const bool inside = a_vec && b_vec && ALAY != 2 && BLAY != 2 && m0 + BM <= p.M && n0 + BN <= p.N && K % BK == 0 &&
+                        m0 % V == 0 && n0 % V == 0;
 
     // step ks computes from LDS buffer ks % 2; (sa_n, sb_n) hold step ks + 1
     // The body has no branches around its loads and stores: a step past the
@@ -526,15 +533,22 @@ __global__ __launch_bounds__(THREADS, (kMinWavesPerEu<T, TM>)) void gemm_mfma_ke
         const int64_t steps = (K + kSplitBK - 1) / kSplitBK, last = steps - 1;
         auto split_run = [&](auto check) {
             constexpr bool CK = decltype(check)::value;
-            ta.template load<CK>(A, p.sam, p.sak, m0, p.M, 0, K);
-            tb.template load<CK>(B, p.sbn, p.sbk, n0, p.N, 0, K);
+            // only a last, partial step of K needs its bounds checked
+            auto load = [&](int64_t k0) {
+                if (CK || k0 + kSplitBK > K) {
+                    ta.template load<true>(A, p.sam, p.sak, m0, p.M, k0, K);
+                    tb.template load<true>(B, p.sbn, p.sbk, n0, p.N, k0, K);
+                } else {
+                    ta.template load<false>(A, p.sam, p.sak, m0, p.M, k0, K);
+                    tb.template load<false>(B, p.sbn, p.sbk, n0, p.N, k0, K);
+                }
+            };
+            load(0);
             for (int64_t s = 0; s < steps; ++s) {
                 ta.store(pa, emin);
                 tb.store(pb, emin);
                 // the next step's loads (the last step's again past the end)
-                const int64_t kn = (s < last ? s + 1 : last) * kSplitBK;
-                ta.template load<CK>(A, p.sam, p.sak, m0, p.M, kn, K);
-                tb.template load<CK>(B, p.sbn, p.sbk, n0, p.N, kn, K);
+                load((s < last ? s + 1 : last) * kSplitBK);
                 __syncthreads();
                 bf16x8 fa[3][TM];
 #pragma unroll
@@ -561,7 +575,7 @@ __global__ __launch_bounds__(THREADS, (kMinWavesPerEu<T, TM>)) void gemm_mfma_ke
                 __syncthreads();
             }
         };
-        if (ALAY != 2 && BLAY != 2 && m0 + BM <= p.M && n0 + BN <= p.N && K % kSplitBK == 0) split_run(std::false_type{});
+        if (ALAY != 2 && BLAY != 2 && m0 + BM <= p.M && n0 + BN <= p.N) split_run(std::false_type{});
         else split_run(std::true_type{});
         bool bad = emin < kSplitMinExp;
 #pragma unroll
@@ -593,7 +607,7 @@ __global__ __launch_bounds__(THREADS, (kMinWavesPerEu<T, TM>)) void gemm_mfma_ke
                 for (int r = 0; r < 4; ++r) {
                     const int64_t m = m0 + wm * WT + i * 16 + M::row(fq, r);
                     const int64_t n = n0 + wn * WT + j * 16 + fr;
-                    if (m < p.M && n < p.N) P[m * p.N + n] = acc[i][j][r];
+                    if (m >= mo && m < p.M && n >= no && n < p.N) P[m * p.N + n] = acc[i][j][r];
                 }
         return;
     }
@@ -641,10 +655,11 @@ __global__ __launch_bounds__(THREADS, (kMinWavesPerEu<T, TM>)) void gemm_mfma_ke
 #pragma unroll
             for (int row = r0; row < QR; row += RS) {
                 const int64_t m = m0 + q * QR + row;
-                if (m >= p.M) continue;
+                if (m < mo || m >= p.M) continue;
                 const VT t = *reinterpret_cast<const VT *>(&tile[row * LDT + V * cg]);
                 const T *tv = reinterpret_cast<const T *>(&t);
-                if (vec && n < p.N) {
+                if (vec) {
+                    if (n < no || n >= p.N) continue;
                     VT rv{};
                     if (resid) rv = *reinterpret_cast<const VT *>(rbase + m * p.srm + n);
                     const T *rr = reinterpret_cast<const T *>(&rv);
@@ -656,7 +671,7 @@ __global__ __launch_bounds__(THREADS, (kMinWavesPerEu<T, TM>)) void gemm_mfma_ke
                 } else {
 #pragma unroll
                     for (int u = 0; u < V; ++u)
-                        if (n + u < p.N) {
+                        if (n + u >= no && n + u < p.N) {
                             const T r = resid ? rbase[m * p.srm + (n + u) * p.srn] : T(0);
                             C[m * p.scm + (n + u) * p.scn] = epilogue_values<T, false>(tv[u], p, bias != nullptr, b[u], r);
                         }
@@ -701,7 +716,7 @@ __global__ __launch_bounds__(THREADS, (kMinWavesPerEu<T, TM>)) void gemm_mfma_ke
             const int col = threadIdx.x % BN;
             const int64_t n = n0 + col;
             const T *bias = static_cast<const T *>(p.nbz ? p.biasz[z0 * p.nb1 + z1] : p.bias);
-            const bool nin = n < p.N, hb = bias != nullptr;
+            const bool nin = n >= no && n < p.N, hb = bias != nullptr;
             const T b = hb && nin ? bias[(p.nbz ? 0 : z0 * p.sbias0 + z1 * p.sbias1) + n * p.sbias] : T(0);
             const T *resid = static_cast<const T *>(p.resid);
             // four rows in flight per thread (4096 x 4096 x 1024 with the
@@ -709,7 +724,7 @@ __global__ __launch_bounds__(THREADS, (kMinWavesPerEu<T, TM>)) void gemm_mfma_ke
 #pragma unroll 4
             for (int row = threadIdx.x / BN; row < QR; row += THREADS / BN) {
                 const int64_t m = m0 + q * QR + row;
-                if (m < p.M && nin) {
+                if (m >= mo && m < p.M && nin) {
                     const T r = resid ? resid[z0 * p.sr0 + z1 * p.sr1 + m * p.srm + n * p.srn] : T(0);
                     C[m * p.scm + n * p.scn] = epilogue_values<T, true>(tile[row * LDT + col], p, hb, b, r, tb);
                 }
@@ -725,8 +740,10 @@ __global__ __launch_bounds__(THREADS, (kMinWavesPerEu<T, TM>)) void gemm_mfma_ke
             for (int r = 0; r < 4; ++r) {
                 const int64_t m = m0 + wm * WT + i * 16 + M::row(fq, r);
                 const int64_t n = n0 + wn * WT + j * 16 + fr;
-                if (m < p.M && n < p.N)
-                    C[m * p.scm + n * p.scn] = gemm_epilogue<T, GELU>(acc[i][j][r], p, z0, z1, m, n);
+                if (m >= mo && m < p.M && n >= no && n < p.N)
+                    // nontemporal: 8192 x 4096 x 64 binary64 120 -> 116 us
+                    __builtin_nontemporal_store(gemm_epilogue<T, GELU>(acc[i][j][r], p, z0, z1, m, n),
+                                                C + m * p.scm + n * p.scn);
             }
 }
 
@@ -846,25 +863,44 @@ void launch_mfma(const GemmProblem &p, dim3 grid, int64_t tm, int64_t tn, bool a
     gemm_mfma_kernel<T, AL, BL, TM, false><<<grid, THREADS, dyn, st>>>(p, tm, tn, av, bv, part, kchunk);
 }
 
-// Slices of K for a product whose tiles cannot fill the chip. 64-tiles:
-// enough slices to give every CU about three workgroups (binary64; two for
-// binary32), each slice at least 256 deep (128 for binary32; a shorter run
-// does not amortize a tile's first loads and its store). (Measured on the skinny f64 8192 x 64 x 4096, 128 64-tiles: 4
-// slices 109.5 us, 6 slices 102.5 us, 8 slices 113.5 us.) 128-tiles (chosen
-// for fewer than two per CU only when K is long, see run_mfma): two
-// workgroups per CU, each slice at least 1024 deep. At most 16 slices;
-// returns 1 for no split.
+// Slices of K for a product whose tiles cannot fill the chip (1: no split),
+// each at least min_depth deep: a shorter run does not amortize a tile's
+// first loads and its store. At most 16 slices. Measured over 1-12 slices, us:
+// 64-tiles, binary32: 1024 x 512 x 784 (128 tiles) 30 unsplit, 22, 22, 20 with
+//   4, 23, 23 with 6; 600 x 512 x 512 (80) 23, 17, 16, 15, 15, 15; 1000^3
+//   (256) 48, 35, 31 with 3, 31; 500 x 4000 x 2000 (504) 97, 81, 87;
+//   2000 x 700 x 300 (352) 23, 24, 26.
+// 64-tiles, binary64: 8192 x 64 x 4096 (128) 182, 104, 104, 86 with 4, 98, 87;
+//   4096 x 64 x 8192 (64) 364, 191, 130, 103, 123, 106, 89 with 8, 95 with 12;
+//   3000 x 500 x 1000 (376) 98, 77 with 2, 84; 3000 x 1000 x 500 (752) 81, 94.
+// 128-tiles, binary32: 4096 x 1024 x 4096 (256) 242, 195 with 2, 205;
+//   1000 x 3000 x 4000 (192) 397, 251, 251, 229, 216 with 5; 500 x 4000 x 2000
+//   (128) 158, 89, 80, 67 with 4, 83.
 template <typename T, int TM>
 int64_t split_count(const GemmProblem &p, int64_t tiles, int64_t *kchunk) {
     constexpr int64_t BK = sizeof(T) == 4 ? kSplitBK : Depth<T, TM>::BK;
     const int64_t cus = device_cus();
-    // 64-tiles, binary32: two workgroups per CU and slices down to 128 deep
-    // (the MLP's 1024 x 512 x 784 product: 4 slices 15.7 us, 3 slices 18.8
-    // us, 6 slices 18.5 us)
-    const int64_t per_cu = TM == 2 ? (sizeof(T) == 4 ? 2 : 3) : 2;
-    const int64_t min_depth = TM == 2 ? (sizeof(T) == 4 ? 128 : 256) : 1024;
-    if (p.causal != 0 || tiles >= (TM == 2 ? cus : 2 * cus) || p.K < 2 * min_depth) return 1;
-    int64_t ks = (per_cu * cus + tiles - 1) / tiles;
+    if (p.causal != 0) return 1;
+    constexpr bool f32 = sizeof(T) == 4;
+    int64_t ks = 1, min_depth = 128;
+    if (TM == 2) {
+        // up to two tiles per CU: slices for two workgroups per CU, or (from
+        // one tile per CU on, where K is worth a combine) for three; binary64
+        // below one and a half
+        if (tiles < cus) ks = (2 * cus + tiles - 1) / tiles;
+        else if (f32 && tiles < 2 * cus && p.K >= 768) ks = (3 * cus + tiles - 1) / tiles;
+        else if (!f32 && 2 * tiles < 3 * cus && p.K >= 768) ks = 2;
+    } else if (tiles < 2 * cus) {
+        // whole rounds of two workgroups per CU: the slice count whose last
+        // round is best filled, least slices first
+        min_depth = f32 ? 512 : 1024;
+        double best = 0;
+        for (int64_t c = 1; c <= 8 && c * min_depth <= p.K; ++c) {
+            const int64_t rounds = (tiles * c + 2 * cus - 1) / (2 * cus);
+            const double fill = (double)(tiles * c) / (double)(rounds * 2 * cus);
+            if (fill > best * 1.12) best = fill, ks = c;
+        }
+    }
     if (ks > p.K / min_depth) ks = p.K / min_depth;
     if (ks > 16) ks = 16;
     if (ks < 2) return 1;
@@ -953,8 +989,12 @@ bool big_tiles(const GemmProblem &p) {
     // 305 us on 64-tiles.
     const int64_t cus = device_cus();
     const int64_t big = ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.nb0 * p.nb1;
-    const int64_t kslices = p.K / 1024 < 16 ? p.K / 1024 : 16;
-    const bool few = big < 2 * cus && !(p.causal == 0 && p.K >= 2048 && big * kslices >= 2 * cus && big >= cus / 2);
+    // binary32 gains from 1024 on: 4096 x 1024 x 1024 65 us as 2 slices
+    // against 68 on 64-tiles, 500 x 4000 x 2000 67 (4 slices) against 81.
+    constexpr bool f32 = sizeof(T) == 4;
+    const int64_t depth = f32 ? 512 : 1024, kslices = p.K / depth < 16 ? p.K / depth : 16;
+    const bool few = big < 2 * cus && !(p.causal == 0 && p.K >= 2 * depth && big >= cus / 2 &&
+                                        (f32 ? 2 * big * kslices >= 3 * cus : big * kslices >= 2 * cus));
     const bool small = few || p.M <= 64 || p.N <= 64 || p.K <= 128;
     return !small;
 }
