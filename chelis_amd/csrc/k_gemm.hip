@@ -371,7 +371,7 @@ __global__ __launch_bounds__(THREADS, (kMinWavesPerEu<T, TM>)) void gemm_mfma_ke
     // (m0, n0), so its loads are the interior tiles' and only the elements of
     // its own it stores. Bounds checks on every load made such tiles the
     // stragglers of the launch: 1000 x 3000 x 4000 with both operands stored
-    // along the outer axis, FIGSHIFT.
+    // along the outer axis, 252 -> 164 us.
     const int64_t mo = (first + in_group % gsz) * BM, no = (in_group / gsz) * BN;
     const int64_t m0 = p.M >= BM && mo + BM > p.M ? p.M - BM : mo, n0 = p.N >= BN && no + BN > p.N ? p.N - BN : no;
     // causal 1: a tile wholly above the diagonal is never read (the whole
@@ -612,7 +612,7 @@ __global__ __launch_bounds__(THREADS, (kMinWavesPerEu<T, TM>)) void gemm_mfma_ke
         return;
     }
     T *C = static_cast<T *>(p.c) + z0 * p.sc0 + z1 * p.sc1;
-    if constexpr (!GELU && sizeof(T) == 4) {
+    if constexpr (!GELU) {
         // The tile through LDS in quarters of BM/4 rows, then each thread
         // finishes V consecutive columns of a row per step - its bias
         // elements read once, residual, output (and the loads) as 16-byte
@@ -620,11 +620,10 @@ __global__ __launch_bounds__(THREADS, (kMinWavesPerEu<T, TM>)) void gemm_mfma_ke
         // each lane would write 64-byte pieces of four rows per store and
         // read the bias and residual an element at a time (measured on
         // 4096 x 4096 x 1024 with a bias: 288 -> 278 us; the transformer
-        // block 974 -> 959 us).
-        constexpr int V = 16 / (int)sizeof(T);
+        // block 974 -> 959 us; binary64 within 1 % either way).
         using VT = typename Vec16<T>::type;
         constexpr int QR = BM / 4, LDT = BN + V, CG = BN / V, RS = THREADS / CG;
-        static_assert(QR * LDT <= 2 * BM * LD, "quarter tile fits in As");
+        static_assert(QR * LDT * sizeof(T) <= sizeof lds, "quarter tile fits");
         T *tile = &As[0][0];
         const int cg = threadIdx.x % CG, r0 = threadIdx.x / CG;
         const int64_t n = n0 + V * cg;
@@ -741,9 +740,7 @@ __global__ __launch_bounds__(THREADS, (kMinWavesPerEu<T, TM>)) void gemm_mfma_ke
                 const int64_t m = m0 + wm * WT + i * 16 + M::row(fq, r);
                 const int64_t n = n0 + wn * WT + j * 16 + fr;
                 if (m >= mo && m < p.M && n >= no && n < p.N)
-                    // nontemporal: 8192 x 4096 x 64 binary64 120 -> 116 us
-                    __builtin_nontemporal_store(gemm_epilogue<T, GELU>(acc[i][j][r], p, z0, z1, m, n),
-                                                C + m * p.scm + n * p.scn);
+                    C[m * p.scm + n * p.scn] = gemm_epilogue<T, GELU>(acc[i][j][r], p, z0, z1, m, n);
             }
 }
 

@@ -53,10 +53,24 @@ constexpr int THREADS = 256, BM = 128, BN = 128, BK = 64, LD = 72;
 // vector of 8 k per row: with the 144-byte row pitch, 16 consecutive lanes
 // write 16 distinct 4-bank groups (rows 4 nb + e, columns 8 kb), where the
 // former element-by-element 2-byte stores took 32 LDS writes per thread.
+// Vectors need only their element's alignment (a global access needs no more
+// on gfx950): a [512, 213] operand is staged as a [512, 216] one.
+typedef uint32_t U4 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t U2 __attribute__((ext_vector_type(2), aligned(2)));
+__device__ inline uint4 load8(const uint16_t *p) {
+    const U4 v = *reinterpret_cast<const U4 *>(p);
+    return uint4{v.x, v.y, v.z, v.w};
+}
+__device__ inline uint2 load4(const uint16_t *p) {
+    const U2 v = *reinterpret_cast<const U2 *>(p);
+    return uint2{v.x, v.y};
+}
+
 template <int LAY, int ROWS>
 struct Stage16 {
     static constexpr int NV = ROWS * BK / 8 / THREADS;
-    static_assert(LAY != 1 || ROWS * BK == 32 * THREADS, "one 4 x 8 block per thread");
+    static_assert(ROWS * BK == 32 * THREADS || ROWS * BK == 16 * THREADS, "a 4 x 8 block per thread, or per other thread");
+    static constexpr int ACTIVE = ROWS * BK / 32;  // LAY 1: threads with a block
     uint4 r[LAY == 1 ? 1 : NV];
     uint2 q[LAY == 1 ? 8 : 1];
 
@@ -67,6 +81,7 @@ struct Stage16 {
                          int64_t k0, int64_t K) {
         const int t = threadIdx.x;
         if constexpr (LAY == 1) {
+            if (ACTIVE < THREADS && t >= ACTIVE) return;
             const int nb = t % 4 + 4 * (t / 32), kb = (t / 4) % 8;
             const int64_t gr = row0 + 4 * nb;
 #pragma unroll
@@ -74,7 +89,7 @@ struct Stage16 {
                 const int64_t gk = k0 + 8 * kb + u;
                 const uint16_t *p = base + gr + gk * s_k;
                 if (!CHECK || (gk < K && gr + 4 <= rows)) {
-                    q[u] = *reinterpret_cast<const uint2 *>(p);
+                    q[u] = load4(p);
                 } else {
                     uint16_t e[4];
 #pragma unroll
@@ -91,7 +106,7 @@ struct Stage16 {
             const int64_t gr = row0 + row, gk = k0 + kv;
             const uint16_t *p = base + gr * s_row + gk * s_k;
             if (LAY == 0 && (!CHECK || (gr < rows && gk + 8 <= K))) {
-                r[j] = *reinterpret_cast<const uint4 *>(p);
+                r[j] = load8(p);
             } else {
                 uint16_t e[8];
 #pragma unroll
@@ -104,6 +119,7 @@ struct Stage16 {
     __device__ void store(uint16_t *lds) const {
         const int t = threadIdx.x;
         if constexpr (LAY == 1) {
+            if (ACTIVE < THREADS && t >= ACTIVE) return;
             const int nb = t % 4 + 4 * (t / 32), kb = (t / 4) % 8;
             // output row e, word w: k = 2w in the low half, 2w + 1 in the high
             uint32_t w[4][4];
@@ -129,8 +145,53 @@ struct Stage16 {
     }
 };
 
-template <Narrow KIND, int ALAY, int BLAY>
+// The finished tile: encoded into LDS (over A's buffers), then written as
+// 16-byte runs of a row where the layout allows. Straight from the
+// accumulators a wave's store is 32-byte pieces of four rows. (With the
+// 64-column tiles: scores and values of 8 x 16 heads of 512 x 64 bf16 61.6 ->
+// 55.4 us, of 4 heads of 64 x 64 18.4 -> 10.9, 56 heads of 777 x 64 f16 165 ->
+// 142. The deep kernel, whose tiles are whole, keeps its direct stores: staged
+// they took 2 x 8 heads of 640 x 128 from 24.8 to 26.7.)
+template <Narrow KIND, int NB>
+__device__ inline void store_tile16(const f32x4 (&acc)[4][NB], uint16_t *tile, uint16_t *C, const GemmProblem &p,
+                                    int64_t m0, int64_t n0) {
+    constexpr int TN = 32 * NB, PITCH = TN + 8, CG = TN / 8;
+    static_assert(BM * PITCH <= 2 * BM * LD, "the tile fits A's buffers");
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, wm = wave >> 1, wn = wave & 1;
+    const int fr = lane & 15, fq = lane >> 4;
+    __syncthreads();  // the main loop's reads are done
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                tile[(wm * 64 + i * 16 + 4 * fq + r) * PITCH + wn * 16 * NB + j * 16 + fr] =
+                    f32_to_narrow<KIND>(acc[i][j][r]);
+    __syncthreads();
+    const int64_t n = n0 + 8 * (t % CG);
+#pragma unroll
+    for (int row = t / CG; row < BM; row += THREADS / CG) {
+        const int64_t m = m0 + row;
+        if (m >= p.M || n >= p.N) continue;
+        const uint16_t *src = tile + row * PITCH + 8 * (t % CG);
+        if (p.scn == 1 && n + 8 <= p.N) {
+            const uint4 q = *reinterpret_cast<const uint4 *>(src);
+            *reinterpret_cast<U4 *>(C + m * p.scm + n) = U4{q.x, q.y, q.z, q.w};
+        } else {
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (n + u < p.N) C[m * p.scm + (n + u) * p.scn] = src[u];
+        }
+    }
+}
+
+// NB: 16-column blocks per wave, 4 for 128-column tiles, 2 for products of
+// at most 64 columns (a head's values: half of a 128-column tile would be
+// padding).
+template <Narrow KIND, int ALAY, int BLAY, int NB>
 __global__ __launch_bounds__(THREADS) void gemm16_kernel(GemmProblem p, int64_t tiles_m, int64_t tiles_n) {
+    constexpr int BN = 32 * NB;
     __shared__ __attribute__((aligned(16))) uint16_t As[2][BM * LD];
     __shared__ __attribute__((aligned(16))) uint16_t Bs[2][BN * LD];
 
@@ -157,11 +218,11 @@ __global__ __launch_bounds__(THREADS) void gemm16_kernel(GemmProblem p, int64_t 
     const int wm = wave >> 1, wn = wave & 1;
     const int fr = lane & 15, fq = lane >> 4;
 
-    f32x4 acc[4][4];
+    f32x4 acc[4][NB];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{};
+        for (int j = 0; j < NB; ++j) acc[i][j] = f32x4{};
 
     Stage16<ALAY, BM> sa;
     Stage16<BLAY, BN> sb;
@@ -184,16 +245,16 @@ __global__ __launch_bounds__(THREADS) void gemm16_kernel(GemmProblem p, int64_t 
 #pragma unroll
             for (int kk = 0; kk < BK / 32; ++kk) {
                 const uint16_t *as = As[buf] + (wm * 64 + fr) * LD + kk * 32 + fq * 8;
-                const uint16_t *bs = Bs[buf] + (wn * 64 + fr) * LD + kk * 32 + fq * 8;
-                uint4 af[4], bf[4];
+                const uint16_t *bs = Bs[buf] + (wn * 16 * NB + fr) * LD + kk * 32 + fq * 8;
+                uint4 af[4], bf[NB];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) af[i] = *reinterpret_cast<const uint4 *>(as + i * 16 * LD);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) bf[j] = *reinterpret_cast<const uint4 *>(bs + j * 16 * LD);
+                for (int j = 0; j < NB; ++j) bf[j] = *reinterpret_cast<const uint4 *>(bs + j * 16 * LD);
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[i][j] = mfma16<KIND>(af[i], bf[j], acc[i][j]);
+                    for (int j = 0; j < NB; ++j) acc[i][j] = mfma16<KIND>(af[i], bf[j], acc[i][j]);
             }
             sa.store(As[buf ^ 1]);
             sb.store(Bs[buf ^ 1]);
@@ -203,17 +264,7 @@ __global__ __launch_bounds__(THREADS) void gemm16_kernel(GemmProblem p, int64_t 
     if (inside) run(std::false_type{});
     else run(std::true_type{});
 
-    uint16_t *C = static_cast<uint16_t *>(p.c) + z0 * p.sc0 + z1 * p.sc1;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int64_t m = m0 + wm * 64 + i * 16 + 4 * fq + r;
-                const int64_t n = n0 + wn * 64 + j * 16 + fr;
-                if (m < p.M && n < p.N) C[m * p.scm + n * p.scn] = f32_to_narrow<KIND>(acc[i][j][r]);
-            }
+    store_tile16<KIND, NB>(acc, As[0], static_cast<uint16_t *>(p.c) + z0 * p.sc0 + z1 * p.sc1, p, m0, n0);
 }
 
 // ---------------------------------------------------------------- deep
@@ -375,18 +426,18 @@ __global__ __launch_bounds__(THREADS, 2) void gemm16_deep_kernel(GemmProblem p, 
 }
 
 // Staging layout of an operand: vectors along K (0) or along its outer
-// axis (1) when that axis has unit stride, the other stride and every batch
-// offset keep 16-byte alignment, and the base is aligned; else 2.
-int lay_of(const void *base, int64_t s_outer, int64_t s_k, int64_t s0, int64_t s1) {
-    const bool aligned = (reinterpret_cast<uintptr_t>(base) & 15u) == 0 && s0 % 8 == 0 && s1 % 8 == 0;
-    if (aligned && s_k == 1 && s_outer % 8 == 0) return 0;
-    if (aligned && s_outer == 1 && s_k % 8 == 0) return 1;
-    return 2;
+// axis (1) where that axis has unit stride, else element by element (2);
+// *aligned: every vector starts on 16 bytes (the deep kernel's).
+int lay_of(const void *base, int64_t s_outer, int64_t s_k, int64_t s0, int64_t s1, bool *aligned) {
+    const bool al = (reinterpret_cast<uintptr_t>(base) & 15u) == 0 && s0 % 8 == 0 && s1 % 8 == 0;
+    *aligned = al && (s_k == 1 ? s_outer : s_k) % 8 == 0;
+    return s_k == 1 ? 0 : s_outer == 1 ? 1 : 2;
 }
 
 template <Narrow KIND, int ALAY, int BLAY>
 void launch16(const GemmProblem &p, dim3 grid, int64_t tm, int64_t tn, hipStream_t st) {
-    gemm16_kernel<KIND, ALAY, BLAY><<<grid, THREADS, 0, st>>>(p, tm, tn);
+    if (p.N <= 64) gemm16_kernel<KIND, ALAY, BLAY, 2><<<grid, THREADS, 0, st>>>(p, tm, tn);
+    else gemm16_kernel<KIND, ALAY, BLAY, 4><<<grid, THREADS, 0, st>>>(p, tm, tn);
 }
 
 template <Narrow KIND>
@@ -395,9 +446,10 @@ int32_t gemm16_kind(const GemmProblem &p, hipStream_t st) {
     const int64_t nz = p.nb0 * p.nb1;
     if (!grid_fits(tm * tn, 256) || nz > 65535) return set_error(CHELIS_HIP_EUNSUPPORTED, "matmul: grid too large");
     const dim3 grid((unsigned)(tm * tn), (unsigned)nz);
-    const int la = lay_of(p.a, p.sam, p.sak, p.sa0, p.sa1), lb = lay_of(p.b, p.sbn, p.sbk, p.sb0, p.sb1);
+    bool aa, ab;
+    const int la = lay_of(p.a, p.sam, p.sak, p.sa0, p.sa1, &aa), lb = lay_of(p.b, p.sbn, p.sbk, p.sb0, p.sb1, &ab);
     // whole tiles and whole steps with A along K: the deep kernel
-    const bool whole = p.M % BM == 0 && p.N % BN == 0 && p.K % BK == 0 && p.K > 0;
+    const bool whole = p.M % BM == 0 && p.N % BN == 0 && p.K % BK == 0 && p.K > 0 && aa && ab;
     if (whole && la == 0 && lb == 0) {
         gemm16_deep_kernel<KIND, 0><<<grid, THREADS, 0, st>>>(p, tm, tn);
         CHELIS_LAUNCH_CHECK();

@@ -196,3 +196,27 @@ def test_narrow_linear_epilogue_unsupported(kind):
     a = C.to_device(carrier(kind, random_bits(kind, (4, 4), 18)))
     with pytest.raises(C.ChelisError, match="no fused epilogue"):
         C.linear(a, a, act="relu")
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("S,D", [(64, 64), (65, 64), (129, 32), (213, 96), (200, 65)])
+def test_narrow_head_products_of_any_length(kind, S, D):
+    """Scores and values of a batch of heads, the operands [B, S, H, D] views:
+    64- and 128-column tiles, partial tiles, rows off 16-byte boundaries and
+    results written whole and in part: within the bound."""
+    B, H = 2, 3
+    q, k, v = (finite_bits(kind, (B, S, H, D), 40 + i) for i in range(3))
+    w = finite_bits(kind, (B, H, S, S), 44)
+    st = (S * H * D, D, H * D, 1)
+    dq, dk, dv = (C.to_device(carrier(kind, t)) for t in (q, k, v))
+    s = C.matmul(dq.view((B, H, S, D), st), dk.view((B, H, D, S), (st[0], st[1], 1, st[2])))
+    o = C.matmul(C.to_device(carrier(kind, w)), dv.view((B, H, S, D), st))
+    at = lambda t, b, h: np.ascontiguousarray(t[b, :, h])
+    for b in range(B):
+        for h in range(H):
+            ref, bound = _mm_bound(kind, at(q, b, h), np.ascontiguousarray(at(k, b, h).T))
+            got = O.narrow_decode(kind, np.ascontiguousarray(bits_of(s.numpy())[b, h])).astype(np.float64)
+            assert np.all(np.abs(got - ref) <= bound)
+            ref, bound = _mm_bound(kind, np.ascontiguousarray(w[b, h]), at(v, b, h))
+            got = O.narrow_decode(kind, np.ascontiguousarray(bits_of(o.numpy())[b, h])).astype(np.float64)
+            assert np.all(np.abs(got - ref) <= bound)
