@@ -53,8 +53,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBPS = 8000.0
-# binary32 products run as six bfloat16 products on the matrix cores
-PEAK_TFLOPS = {"f32": 2500.0 / 6, "f64": 78.6, "bf16": 2500.0}
+PEAK_TFLOPS = {"f32": 157.3, "f64": 78.6, "bf16": 2500.0}
 METRIC = "per-kernel GB/s & GFLOP/s (% roofline); transformer-block fwd ms at 1 GPU"
 SOFTMAX_ROWS, SOFTMAX_N = 16384, 1024
 

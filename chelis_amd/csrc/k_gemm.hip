@@ -1,8 +1,7 @@
 // Dense matmul on the CDNA4 matrix cores, and the matmul / linear entry
 // points with their shape dispatch.
 //
-// MFMA tile kernel (binary64; binary32 multiplies in bfloat16 pieces, see
-// below, and falls back to this loop). A 256-thread workgroup (4 waves, 2 x 2) owns a 128 x 128
+// MFMA tile kernel. A 256-thread workgroup (4 waves, 2 x 2) owns a 128 x 128
 // tile of C; each wave owns 64 x 64 = 4 x 4 blocks of 16 x 16, accumulated
 // by v_mfma_f32_16x16x4_f32 (f32) or v_mfma_f64_16x16x4_f64 (f64); a 64 x 64
 // tile (32 x 32 per wave) serves products with few 128-tiles. K moves in
@@ -203,136 +202,11 @@ struct Stage {
     }
 };
 
-// ---------------------------------------------------------------- binary32 in three bfloat16 pieces
-// A binary32 value is exactly the sum of three bfloat16 values, x = h + m + l
-// (each the remainder rounded to nearest: 8 + 8 + 8 significant bits), and
-// a product of two of them is exact in binary32, so
-//   x y = h h' + (h m' + m h') + (h l' + m m' + l h') + dropped
-// with the dropped m l', l m' and l l' within 2^-26 of x y: six bfloat16
-// products (v_mfma_f32_16x16x32_bf16, sixteen times the binary32 matrix
-// rate) with a binary32 accumulator in place of one binary32 product. The
-// accumulator is rounded once per product of 32 terms, six times per 32
-// terms in all, against 32 times on v_mfma_f32_16x16x4_f32, so the sum is
-// closer to the exact one, not further: the relative 2-norm error against
-// binary64 of 512 x 512 x K products of normal values is 6.5e-8, 1.5e-7,
-// 1.6e-7, 3.5e-7 at K = 33, 128, 1024, 4096, against 1.05e-7, 2.0e-7, 2.1e-7,
-// 4.1e-7 on v_mfma_f32_16x16x4_f32, and lower at every K tried, for uniform
-// values too. 4096^3: 1046 -> 724 us (190 TFLOP/s of binary32 products,
-// 1.14 PFLOP/s on the bfloat16 cores); 4096 x 4096 x 1024 with a bias 279
-// -> 198 us. Of the 724, 30 are the exponent test (without it 694).
-// The pieces are exact while every piece is a normal number: 0 or |x| at
-// least 2^-103. A tile that met a smaller value, or whose sums are not all
-// finite (an infinity or NaN has no such pieces, and a value near the
-// largest rounds to one), is computed again by the binary32 loop.
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-
-constexpr int kSplitBK = 32;           // K per step: one MFMA
-constexpr int kSplitLD = kSplitBK + 8; // LDS row pitch, 80 bytes: 16 rows of one read on 64 banks
-constexpr int kSplitMinExp = -102;     // frexp exponent of the least magnitude split exactly
-
-__device__ inline uint32_t pack_bf16(float a, float b) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
-}
-// The pieces of N (2 or 4) values, two to a word.
-template <int N>
-__device__ inline void split_bf16(const float (&x)[N], uint32_t (&h)[N / 2], uint32_t (&m)[N / 2],
-                                  uint32_t (&l)[N / 2], int &emin) {
-#pragma unroll
-    for (int i = 0; i < N / 2; ++i) {
-        const float a = x[2 * i], b = x[2 * i + 1];
-        const int ea = __builtin_amdgcn_frexp_expf(a), eb = __builtin_amdgcn_frexp_expf(b);
-        const int e = ea < eb ? ea : eb;
-        emin = e < emin ? e : emin;
-        h[i] = pack_bf16(a, b);
-        const float ra = a - f32_from(h[i] << 16), rb = b - f32_from(h[i] & 0xffff0000u);
-        m[i] = pack_bf16(ra, rb);
-        l[i] = pack_bf16(ra - f32_from(m[i] << 16), rb - f32_from(m[i] & 0xffff0000u));
-    }
-}
-
-// One operand's step of a tile: [ROWS][32] binary32 values staged in
-// registers, then split into the three planes of LDS (K-contiguous rows).
-// LAY as for Stage: 0 four consecutive k of a row per vector, 1 four rows of
-// one k per vector (transposed in registers), 2 element by element. Vectors
-// need only their element's alignment.
-template <int LAY, int ROWS>
-struct StageSplit {
-    static constexpr int BK = kSplitBK, NE = ROWS * BK / THREADS;
-    static constexpr int KU = LAY == 1 ? NE / 4 : 4, RU = NE / KU;  // a thread's k and rows
-    typedef float F4 __attribute__((ext_vector_type(4), aligned(4)));
-    float r[RU][KU];
-
-    __device__ static int row_of(int u) {
-        const int t = threadIdx.x;
-        if constexpr (LAY == 1) return (t / (BK / KU)) * 4 + u;
-        else return t / 8 + (THREADS / 8) * u;
-    }
-    __device__ static int k_of() {
-        if constexpr (LAY == 1) return (threadIdx.x % (BK / KU)) * KU;
-        else return (threadIdx.x % 8) * 4;
-    }
-    template <bool CHECK>
-    __device__ void load(const float *__restrict__ base, int64_t s_row, int64_t s_k, int64_t row0, int64_t rows,
-                         int64_t k0, int64_t K) {
-        const int64_t gk = k0 + k_of();
-        if constexpr (LAY == 1) {
-            const int64_t gr = row0 + row_of(0);
-#pragma unroll
-            for (int k = 0; k < KU; ++k) {
-                const float *p = base + gr + (gk + k) * s_k;
-                if (!CHECK || (gk + k < K && gr + 4 <= rows)) {
-                    const F4 q = *reinterpret_cast<const F4 *>(p);
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) r[u][k] = q[u];
-                } else {
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) r[u][k] = gk + k < K && gr + u < rows ? p[u] : 0.0f;
-                }
-            }
-        } else {
-#pragma unroll
-            for (int u = 0; u < RU; ++u) {
-                const int64_t gr = row0 + row_of(u);
-                const float *p = base + gr * s_row + gk * s_k;
-                if (LAY == 0 && (!CHECK || (gr < rows && gk + 4 <= K))) {
-                    const F4 q = *reinterpret_cast<const F4 *>(p);
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) r[u][k] = q[k];
-                } else {
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) r[u][k] = gr < rows && gk + k < K ? p[k * s_k] : 0.0f;
-                }
-            }
-        }
-    }
-    // planes: [3][ROWS][kSplitLD]
-    __device__ void store(uint16_t *planes, int &emin) const {
-        constexpr int P = ROWS * kSplitLD;
-#pragma unroll
-        for (int u = 0; u < RU; ++u) {
-            uint16_t *d = planes + row_of(u) * kSplitLD + k_of();
-            uint32_t h[KU / 2], m[KU / 2], l[KU / 2];
-            split_bf16<KU>(r[u], h, m, l, emin);
-            if constexpr (KU == 4) {
-                *reinterpret_cast<uint2 *>(d) = uint2{h[0], h[1]};
-                *reinterpret_cast<uint2 *>(d + P) = uint2{m[0], m[1]};
-                *reinterpret_cast<uint2 *>(d + 2 * P) = uint2{l[0], l[1]};
-            } else {
-                *reinterpret_cast<uint32_t *>(d) = h[0];
-                *reinterpret_cast<uint32_t *>(d + P) = m[0];
-                *reinterpret_cast<uint32_t *>(d + 2 * P) = l[0];
-            }
-        }
-    }
-};
-
 // f64 holds its 64x64 accumulators in 128 registers; capping the kernel at
 // 256 registers per lane keeps two waves per SIMD resident (measured 1.6x
 // over one wave at 4096^3). f32 is fastest with the compiler's own choice.
-template <typename T, int TM>
-constexpr int kMinWavesPerEu = sizeof(T) == 8 || TM == 4 ? 2 : 3;
+template <typename T>
+constexpr int kMinWavesPerEu = sizeof(T) == 8 ? 2 : 1;
 
 // TM = 16x16 blocks per wave and dimension: 4 gives the 128 x 128 tile for
 // large products, 2 a 64 x 64 tile for products with few 128-tiles.
@@ -340,7 +214,7 @@ constexpr int kMinWavesPerEu = sizeof(T) == 8 || TM == 4 ? 2 : 3;
 // BK) and each slice stores its raw sums to part[slice][z][m][n]; a combine
 // pass adds the slices in slice order and applies the epilogue.
 template <typename T, int ALAY, int BLAY, int TM, bool GELU>
-__global__ __launch_bounds__(THREADS, (kMinWavesPerEu<T, TM>)) void gemm_mfma_kernel(GemmProblem p, int64_t tiles_m,
+__global__ __launch_bounds__(THREADS, kMinWavesPerEu<T>) void gemm_mfma_kernel(GemmProblem p, int64_t tiles_m,
                                                                                int64_t tiles_n, bool a_vec,
                                                                                bool b_vec, T *part,
                                                                                int64_t kchunk) {
@@ -349,13 +223,9 @@ __global__ __launch_bounds__(THREADS, (kMinWavesPerEu<T, TM>)) void gemm_mfma_ke
     using D = Depth<T, TM>;
     constexpr int BK = D::BK, LD = D::LD, KV = D::KV, V = M::V, NVF = KV / V;
     constexpr int BM = 32 * TM, BN = 32 * TM, WT = 16 * TM;
-    // the binary32 or binary64 loop's buffers, and over them (binary32) the
-    // three planes of each operand
-    constexpr size_t kTile = 2 * sizeof(T) * (BM + BN) * LD;
-    constexpr size_t kPlanes = sizeof(T) == 4 ? 2 * 3 * (BM + BN) * kSplitLD : 0;
-    __shared__ __attribute__((aligned(16))) unsigned char lds[kTile > kPlanes ? kTile : kPlanes];
+    __shared__ __attribute__((aligned(16))) T lds[2 * (BM + BN) * LD];
     T(*As)[BM * LD] = reinterpret_cast<T(*)[BM * LD]>(lds);
-    T(*Bs)[BN * LD] = reinterpret_cast<T(*)[BN * LD]>(lds + 2 * sizeof(T) * BM * LD);
+    T(*Bs)[BN * LD] = reinterpret_cast<T(*)[BN * LD]>(lds + 2 * BM * LD);
 
     // XCD-aware tile order.
     const int64_t tiles = tiles_m * tiles_n;
@@ -371,7 +241,7 @@ __global__ __launch_bounds__(THREADS, (kMinWavesPerEu<T, TM>)) void gemm_mfma_ke
     // (m0, n0), so its loads are the interior tiles' and only the elements of
     // its own it stores. Bounds checks on every load made such tiles the
     // stragglers of the launch: 1000 x 3000 x 4000 with both operands stored
-    // along the outer axis, 252 -> 164 us.
+    // along the outer axis, 338 -> 266 us.
     const int64_t mo = (first + in_group % gsz) * BM, no = (in_group / gsz) * BN;
     const int64_t m0 = p.M >= BM && mo + BM > p.M ? p.M - BM : mo, n0 = p.N >= BN && no + BN > p.N ? p.N - BN : no;
     // causal 1: a tile wholly above the diagonal is never read (the whole
@@ -522,80 +392,8 @@ __global__ __launch_bounds__(THREADS, (kMinWavesPerEu<T, TM>)) void gemm_mfma_ke
             if (ks < ksteps) step(ks, f0, f1, sa0, sb0);
         }
     };
-    bool redo = true;
-    if constexpr (sizeof(T) == 4) {
-        // one buffer of planes: the other workgroup of the CU fills the
-        // matrix cores while this one splits and stores
-        uint16_t *pa = reinterpret_cast<uint16_t *>(lds), *pb = pa + 3 * BM * kSplitLD;
-        StageSplit<ALAY, BM> ta;
-        StageSplit<BLAY, BN> tb;
-        int emin = 0;
-        const int64_t steps = (K + kSplitBK - 1) / kSplitBK, last = steps - 1;
-        auto split_run = [&](auto check) {
-            constexpr bool CK = decltype(check)::value;
-            // only a last, partial step of K needs its bounds checked
-            auto load = [&](int64_t k0) {
-                if (CK || k0 + kSplitBK > K) {
-                    ta.template load<true>(A, p.sam, p.sak, m0, p.M, k0, K);
-                    tb.template load<true>(B, p.sbn, p.sbk, n0, p.N, k0, K);
-                } else {
-                    ta.template load<false>(A, p.sam, p.sak, m0, p.M, k0, K);
-                    tb.template load<false>(B, p.sbn, p.sbk, n0, p.N, k0, K);
-                }
-            };
-            load(0);
-            for (int64_t s = 0; s < steps; ++s) {
-                ta.store(pa, emin);
-                tb.store(pb, emin);
-                // the next step's loads (the last step's again past the end)
-                load((s < last ? s + 1 : last) * kSplitBK);
-                __syncthreads();
-                bf16x8 fa[3][TM];
-#pragma unroll
-                for (int h = 0; h < 3; ++h)
-#pragma unroll
-                    for (int i = 0; i < TM; ++i)
-                        fa[h][i] = *reinterpret_cast<const bf16x8 *>(pa + (h * BM + wm * WT + i * 16 + fr) * kSplitLD +
-                                                                     fq * 8);
-#pragma unroll
-                for (int j = 0; j < TM; ++j) {
-                    bf16x8 fb[3];
-#pragma unroll
-                    for (int h = 0; h < 3; ++h)
-                        fb[h] = *reinterpret_cast<const bf16x8 *>(pb + (h * BN + wn * WT + j * 16 + fr) * kSplitLD +
-                                                                  fq * 8);
-                    // smallest terms first, the wave's TM sums in turn
-                    constexpr int ha[6] = {0, 1, 2, 0, 1, 0}, hb[6] = {2, 1, 0, 1, 0, 0};
-#pragma unroll
-                    for (int q = 0; q < 6; ++q)
-#pragma unroll
-                        for (int i = 0; i < TM; ++i)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[ha[q]][i], fb[hb[q]], acc[i][j], 0, 0, 0);
-                }
-                __syncthreads();
-            }
-        };
-        if (ALAY != 2 && BLAY != 2 && m0 + BM <= p.M && n0 + BN <= p.N) split_run(std::false_type{});
-        else split_run(std::true_type{});
-        bool bad = emin < kSplitMinExp;
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TM; ++j)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) bad = bad || !__builtin_isfinite(acc[i][j][r]);
-        redo = __syncthreads_or(bad);
-        if (redo) {
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TM; ++j) acc[i][j] = acc_t{};
-        }
-    }
-    if (redo) {
-        if (inside) run(std::false_type{});
-        else run(std::true_type{});
-    }
+    if (inside) run(std::false_type{});
+    else run(std::true_type{});
 
     if (kchunk > 0) {
         T *P = part + ((int64_t)blockIdx.z * gridDim.y + z) * p.M * p.N;
@@ -832,18 +630,6 @@ int lay_of(int64_t s_outer, int64_t s_k, const void *base, int64_t outer, int64_
     return 2;
 }
 
-// Occupancy of the f32 128-tile kernel without the GELU epilogue: its 40 KiB
-// of LDS allow three workgroups per CU. Its registers decide first: the
-// current build holds 224 per lane (116 vector + 108 accumulation), two
-// waves per SIMD, so two workgroups per CU. Were the count to drop to 168 or
-// fewer, a grid of T tiles would run in ceil(T / 3C) rounds of three; two
-// per CU (ceil(T / 2C) rounds of two) is then kept when that is fewer
-// workgroup-slots in all, e.g. 1024 tiles on 256 CUs as two full rounds of
-// two rather than a round of three and a third of one (measured 1.42 ms
-// against 1.54 ms at 4096^3 with an earlier build that fitted three).
-// Dynamic LDS beyond a third of the CU's 160 KiB pins two.
-constexpr size_t kPinTwoLds = 16384;
-
 template <typename T, int AL, int BL, int TM>
 void launch_mfma(const GemmProblem &p, dim3 grid, int64_t tm, int64_t tn, bool av, bool bv, T *part, int64_t kchunk,
                  hipStream_t st) {
@@ -852,40 +638,31 @@ void launch_mfma(const GemmProblem &p, dim3 grid, int64_t tm, int64_t tn, bool a
         gemm_mfma_kernel<T, AL, BL, TM, true><<<grid, THREADS, 0, st>>>(p, tm, tn, av, bv, part, kchunk);
         return;
     }
-    size_t dyn = 0;
-    if (sizeof(T) == 4 && TM == 4) {
-        const int64_t C = device_cus(), t = (int64_t)grid.x * grid.y * grid.z;
-        if (((t + 2 * C - 1) / (2 * C)) * 2 <= ((t + 3 * C - 1) / (3 * C)) * 3) dyn = kPinTwoLds;
-    }
-    gemm_mfma_kernel<T, AL, BL, TM, false><<<grid, THREADS, dyn, st>>>(p, tm, tn, av, bv, part, kchunk);
+    gemm_mfma_kernel<T, AL, BL, TM, false><<<grid, THREADS, 0, st>>>(p, tm, tn, av, bv, part, kchunk);
 }
 
 // Slices of K for a product whose tiles cannot fill the chip (1: no split),
 // each at least min_depth deep: a shorter run does not amortize a tile's
 // first loads and its store. At most 16 slices. Measured over 1-12 slices, us:
-// 64-tiles, binary32: 1024 x 512 x 784 (128 tiles) 30 unsplit, 22, 22, 20 with
-//   4, 23, 23 with 6; 600 x 512 x 512 (80) 23, 17, 16, 15, 15, 15; 1000^3
-//   (256) 48, 35, 31 with 3, 31; 500 x 4000 x 2000 (504) 97, 81, 87;
-//   2000 x 700 x 300 (352) 23, 24, 26.
+// 64-tiles, binary32: 1024 x 512 x 784 (128 tiles) 33 unsplit, 24, 24, 21.6
+//   with 4, 25; 600 x 512 x 2048 (80) 50, 30, 24, 28, 25, 24 with 6, 26 with 8;
+//   500 x 4000 x 2000 (504) 111, 97; 2000 x 700 x 300 (352) 25, 27.
 // 64-tiles, binary64: 8192 x 64 x 4096 (128) 182, 104, 104, 86 with 4, 98, 87;
 //   4096 x 64 x 8192 (64) 364, 191, 130, 103, 123, 106, 89 with 8, 95 with 12;
 //   3000 x 500 x 1000 (376) 98, 77 with 2, 84; 3000 x 1000 x 500 (752) 81, 94.
-// 128-tiles, binary32: 4096 x 1024 x 4096 (256) 242, 195 with 2, 205;
-//   1000 x 3000 x 4000 (192) 397, 251, 251, 229, 216 with 5; 500 x 4000 x 2000
-//   (128) 158, 89, 80, 67 with 4, 83.
+// 128-tiles, binary32: 4096 x 1024 x 4096 (256) 302, 277 with 2, 289;
+//   1000 x 3000 x 4000 (192) 294, 267, 273, 215 with 4, 227 with 5.
 template <typename T, int TM>
 int64_t split_count(const GemmProblem &p, int64_t tiles, int64_t *kchunk) {
-    constexpr int64_t BK = sizeof(T) == 4 ? kSplitBK : Depth<T, TM>::BK;
+    constexpr int64_t BK = Depth<T, TM>::BK;
     const int64_t cus = device_cus();
     if (p.causal != 0) return 1;
     constexpr bool f32 = sizeof(T) == 4;
     int64_t ks = 1, min_depth = 128;
     if (TM == 2) {
-        // up to two tiles per CU: slices for two workgroups per CU, or (from
-        // one tile per CU on, where K is worth a combine) for three; binary64
-        // below one and a half
+        // below a tile per CU: slices for two workgroups per CU; binary64 up
+        // to one and a half tiles per CU: two slices
         if (tiles < cus) ks = (2 * cus + tiles - 1) / tiles;
-        else if (f32 && tiles < 2 * cus && p.K >= 768) ks = (3 * cus + tiles - 1) / tiles;
         else if (!f32 && 2 * tiles < 3 * cus && p.K >= 768) ks = 2;
     } else if (tiles < 2 * cus) {
         // whole rounds of two workgroups per CU: the slice count whose last
@@ -986,12 +763,8 @@ bool big_tiles(const GemmProblem &p) {
     // 305 us on 64-tiles.
     const int64_t cus = device_cus();
     const int64_t big = ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.nb0 * p.nb1;
-    // binary32 gains from 1024 on: 4096 x 1024 x 1024 65 us as 2 slices
-    // against 68 on 64-tiles, 500 x 4000 x 2000 67 (4 slices) against 81.
-    constexpr bool f32 = sizeof(T) == 4;
-    const int64_t depth = f32 ? 512 : 1024, kslices = p.K / depth < 16 ? p.K / depth : 16;
-    const bool few = big < 2 * cus && !(p.causal == 0 && p.K >= 2 * depth && big >= cus / 2 &&
-                                        (f32 ? 2 * big * kslices >= 3 * cus : big * kslices >= 2 * cus));
+    const int64_t kslices = p.K / 1024 < 16 ? p.K / 1024 : 16;
+    const bool few = big < 2 * cus && !(p.causal == 0 && p.K >= 2048 && big * kslices >= 2 * cus && big >= cus / 2);
     const bool small = few || p.M <= 64 || p.N <= 64 || p.K <= 128;
     return !small;
 }

@@ -361,9 +361,8 @@ int32_t chelis_hip_relu_adjoint(const chelis_gpu_tensor *x, const chelis_gpu_ten
  * and b (a transposed operand is a stride swap, never a copy; up to two
  * batch axes broadcast numpy-style, an extent-1 axis by stride 0; a rank-1
  * a is a row [1, K] and a rank-1 b a column [K, 1], their axis dropped from
- * c) and c any non-overlapping view. Dense shapes run on MFMA (binary32 as
- * three bfloat16 pieces per operand, within the binary32 sum's error, on
- * v_mfma_f32_16x16x32_bf16; v_mfma_f64_16x16x4_f64); short K (<= 32), GEMV
+ * c) and c any non-overlapping view. Dense shapes run on MFMA
+ * (v_mfma_f32_16x16x4_f32 / v_mfma_f64_16x16x4_f64); short K (<= 32), GEMV
  * (M or N == 1) and skinny shapes (min(M, N) < 16, or <= 64 in f64) run on
  * VALU kernels whose K sum is the canonical tree, bit-exact with the C lane.
  * `flags` = CHELIS_MATMUL_EXACT forces the canonical-tree kernels on every

@@ -467,10 +467,10 @@ def _binary32_bound(a, b):
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt", "strided"])
 @pytest.mark.parametrize("shape", [(16, 16, 33), (64, 64, 64), (65, 130, 100), (129, 257, 1000), (640, 2048, 96),
                                    (1100, 3000, 161)])
-def test_binary32_pieces_at_the_tile_edges(shape, layout):
-    """Binary32 products on the bfloat16 cores (three pieces per value): whole
-    and partial tiles and K steps, 64- and 128-tiles, every staging layout,
-    rows off 16-byte boundaries; within the binary32 bound."""
+def test_binary32_products_at_the_tile_edges(shape, layout):
+    """Binary32 products: whole and partial tiles and K steps, 64- and
+    128-tiles, every staging layout, rows off 16-byte boundaries; within the
+    binary32 bound, elementwise."""
     M, N, K = shape
     rng = np.random.default_rng(M + N + K)
     a, b = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, N)).astype(np.float32)
@@ -488,9 +488,9 @@ def test_binary32_pieces_at_the_tile_edges(shape, layout):
 
 
 @pytest.mark.parametrize("sa,sb", [(1e-36, 1.0), (1e-42, 1e30), (1.0, 1e-40), (1e-20, 1e-22), (1e18, 1e18)])
-def test_binary32_pieces_at_the_ends_of_the_range(sa, sb):
-    """Operands whose pieces would fall below the normal numbers (computed by
-    the binary32 loop), sums among the subnormals, and sums near the top."""
+def test_binary32_products_at_the_ends_of_the_range(sa, sb):
+    """Operands among the smallest numbers, sums among the subnormals, and
+    sums near the top."""
     rng = np.random.default_rng(3)
     a = (rng.uniform(0.5, 1, (200, 160)) * sa).astype(np.float32)
     b = (rng.uniform(-1, 1, (160, 136)) * sb).astype(np.float32)
@@ -500,10 +500,10 @@ def test_binary32_pieces_at_the_ends_of_the_range(sa, sb):
     assert (np.abs(c - ref) <= bound).all(), float((np.abs(c - ref) / bound).max())
 
 
-def test_binary32_pieces_infinities_nan_and_the_largest_values():
+def test_binary32_products_infinities_nan_and_the_largest_values():
     """An infinity or a NaN reaches the rows and columns it belongs to and no
-    other, a value that rounds past the largest bfloat16 stays exact, and sums
-    past the range are infinite: as the binary32 products give them."""
+    other, the largest value stays exact, and sums past the range are
+    infinite."""
     rng = np.random.default_rng(4)
     a = rng.standard_normal((200, 64)).astype(np.float32)
     b = rng.uniform(0.5, 1, (64, 200)).astype(np.float32)
@@ -515,3 +515,65 @@ def test_binary32_pieces_infinities_nan_and_the_largest_values():
     rest = np.delete(np.arange(200), [3, 70, 131])
     ref, bound = _binary32_bound(a[rest], b)
     assert (np.abs(c[rest] - ref) <= bound).all()
+
+
+# products that take 64-tiles, 64-tiles cut along K, 128-tiles, 128-tiles cut
+# along K, and partial tiles and K steps of each
+TILED = [(200, 160, 136), (600, 512, 520), (1100, 3000, 161), (500, 1500, 2080), (2100, 2050, 1030)]
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("shape", TILED)
+def test_binary32_sums_of_one_term_are_correctly_rounded(shape, layout):
+    """One nonzero per row of A: every result is one product, rounded once."""
+    M, N, K = shape
+    rng = np.random.default_rng(M + K)
+    a = np.zeros((M, K), np.float32)
+    at = rng.integers(0, K, M)
+    a[np.arange(M), at] = rng.standard_normal(M).astype(np.float32)
+    b = rng.standard_normal((K, N)).astype(np.float32)
+    da, db = (dev_view(x, *x.shape, t == "t")[:2] for x, t in ((a, layout[0]), (b, layout[1])))
+    c = C.matmul(da[1], db[1]).numpy()
+    assert bits_equal(c, a[np.arange(M), at][:, None] * b[at])
+
+
+@pytest.mark.parametrize("shape", TILED + [(512, 512, 20000)])
+@pytest.mark.parametrize("positive", [False, True])
+def test_binary32_sums_in_the_two_norm(shape, positive):
+    """The 2-norm error against binary64 of K roundings at random: a rounding
+    of a running sum of k terms errs by 0.43 x 2^-24 of it (rms, the mantissas
+    spread over their logarithm), so normal terms, whose sums grow as sqrt(k),
+    err by 0.43 x 2^-24 sqrt(K / 2) of the result, and positive ones, whose
+    sums grow as k, by 0.43 x 2^-24 sqrt(K / 3). A quarter above that, and a
+    rounding of the result, are allowed: 16-bit significands (2^-17) or a
+    rounding in one direction (K 2^-25) are far outside."""
+    M, N, K = shape
+    rng = np.random.default_rng(N + K)
+    draw = rng.random if positive else rng.standard_normal
+    a, b = draw((M, K)).astype(np.float32), draw((K, N)).astype(np.float32)
+    c = C.matmul(C.to_device(a), C.to_device(b)).numpy().astype(np.float64)
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    err = np.linalg.norm(c - ref) / np.linalg.norm(ref)
+    assert err <= 2.0 ** -24 * (1.25 * 0.43 * np.sqrt(K / (3 if positive else 2)) + 0.5), err * 2.0 ** 24
+
+
+@pytest.mark.parametrize("layout", ["nn", "tn"])
+@pytest.mark.parametrize("shape", TILED)
+@pytest.mark.parametrize("act", [None, "gelu"])
+def test_binary32_rows_do_not_depend_on_their_neighbours(shape, layout, act):
+    """An infinity, a NaN, the largest value and subnormal values in some rows
+    of A and columns of B leave every other result's bits alone."""
+    M, N, K = shape
+    rng = np.random.default_rng(M + N)
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    b = rng.uniform(0.5, 1, (K, N)).astype(np.float32)
+    run = lambda x: C.linear(dev_view(x, M, K, layout[0] == "t")[1], C.to_device(b), act=act).numpy()
+    want = run(a)
+    rows, cols = np.array([1, M // 3, M // 2, M - 2]), np.array([3, N - 1])
+    for r, v, k in zip(rows, (np.inf, np.nan, np.float32(3.4e38), np.float32(1e-40)), (0, K // 2, K - 1, K // 3)):
+        a[r, k] = v
+    b[K // 2, cols[0]], b[K - 1, cols[1]] = np.float32(1e-42), np.inf
+    got = run(a)
+    keep = np.ix_(np.delete(np.arange(M), rows), np.delete(np.arange(N), cols))
+    assert bits_equal(got[keep], want[keep])
+    assert np.isnan(got[rows[1]]).all()
