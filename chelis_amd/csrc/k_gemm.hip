@@ -647,9 +647,11 @@ void launch_mfma(const GemmProblem &p, dim3 grid, int64_t tm, int64_t tn, bool a
 // 64-tiles, binary32: 1024 x 512 x 784 (128 tiles) 33 unsplit, 24, 24, 21.6
 //   with 4, 25; 600 x 512 x 2048 (80) 50, 30, 24, 28, 25, 24 with 6, 26 with 8;
 //   500 x 4000 x 2000 (504) 111, 97; 2000 x 700 x 300 (352) 25, 27.
-// 64-tiles, binary64: 8192 x 64 x 4096 (128) 182, 104, 104, 86 with 4, 98, 87;
-//   4096 x 64 x 8192 (64) 364, 191, 130, 103, 123, 106, 89 with 8, 95 with 12;
-//   3000 x 500 x 1000 (376) 98, 77 with 2, 84; 3000 x 1000 x 500 (752) 81, 94.
+// 64-tiles, binary64 (B along N; K-contiguous both; A along M): 8192 x 64 x
+//   4096 (128) 182 unsplit, 99, 103, 90.4; 88.1; 86.0 with 4, 86.4; 84.1; 89.9
+//   with 6, 98 with 8; 4096 x 64 x 8192 (64) 85.7; 84.2; 85.9 with 8, 86.0;
+//   83.9; 89.8 with 12; 512 x 512 x 4096 (64) 47.6 with 8, 49.8 with 12; 3000 x
+//   500 x 1000 (376) 103, 79 with 2, 85; 500 x 4000 x 2000 (504) 140, 145.
 // 128-tiles, binary32: 4096 x 1024 x 4096 (256) 302, 277 with 2, 289;
 //   1000 x 3000 x 4000 (192) 294, 267, 273, 215 with 4, 227 with 5.
 template <typename T, int TM>
@@ -660,9 +662,11 @@ int64_t split_count(const GemmProblem &p, int64_t tiles, int64_t *kchunk) {
     constexpr bool f32 = sizeof(T) == 4;
     int64_t ks = 1, min_depth = 128;
     if (TM == 2) {
-        // below a tile per CU: slices for two workgroups per CU; binary64 up
-        // to one and a half tiles per CU: two slices
-        if (tiles < cus) ks = (2 * cus + tiles - 1) / tiles;
+        // below a tile per CU: slices for two workgroups per CU, or (binary64
+        // slices that stay 640 deep) for three; binary64 up to one and a half
+        // tiles per CU: two slices
+        const int64_t three = (3 * cus + tiles - 1) / tiles;
+        if (tiles < cus) ks = !f32 && p.K / three >= 640 ? three : (2 * cus + tiles - 1) / tiles;
         else if (!f32 && 2 * tiles < 3 * cus && p.K >= 768) ks = 2;
     } else if (tiles < 2 * cus) {
         // whole rounds of two workgroups per CU: the slice count whose last
