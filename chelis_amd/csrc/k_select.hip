@@ -1507,9 +1507,14 @@ extern "C" int32_t chelis_hip_pad(const chelis_gpu_tensor *x, const int64_t *lo,
 }
 
 namespace {
-// Rows of at least 16 columns take the row kernels; narrower ones (and
-// ScatterElements) a lane per element.
-bool scatter_by_rows(int32_t mode, const ScatterGeom &g) { return mode != 2 && g.after >= 16; }
+// Rows of at least 16 columns take the row kernels; narrower ones,
+// ScatterElements, and more rows than one launch of a wave per row and 64
+// columns holds (2^26 - 4 rows of up to 64 columns), a lane per element.
+bool scatter_by_rows(int32_t mode, const ScatterGeom &g) {
+    if (mode == 2 || g.after < 16) return false;
+    const int64_t n = g.total / g.after, chunks = (g.after + 63) / 64;
+    return grid_fits((n * chunks + 3) / 4, 256) && grid_fits((n + 15) / 16 * chunks, 256);
+}
 
 // out = target: nothing when they are one tensor, a dense copy where both
 // are contiguous whole dwords, else the strided copy of pad.
@@ -1544,8 +1549,6 @@ int32_t run_scatter(int32_t mode, const chelis_gpu_tensor *target, const chelis_
     kg.span = after;
     if (rows) kg.after = 1, kg.total = n;
     const int64_t chunks = (after + 63) / 64;
-    if (rows && (!grid_fits((n * chunks + 3) / 4, 256) || !grid_fits((n + 15) / 16 * chunks, 256)))
-        return set_error(CHELIS_HIP_EUNSUPPORTED, "scatter: too many rows of updates");
     int end_bit = 1;
     while (end_bit < (int)(8 * sizeof(K)) && ((uint64_t)sentinel >> end_bit) != 0) ++end_bit;
     size_t temp = 0;

@@ -557,3 +557,20 @@ def test_gather_rows_of_whole_and_partial_vectors(dtype, after):
     want, first = O.gather(values, idx, 1, 1)[:2]
     got, failure = C.gather(C.to_device(values), C.to_device(idx), 1, 1)
     assert failure[0] == first and got.numpy().tobytes() == want.tobytes()
+
+
+@pytest.mark.parametrize("add", [False, True])
+def test_scatter_of_more_rows_than_one_launch_of_waves(add):
+    """2^26 - 3 rows of 16 columns, one more than the row kernels' launch
+    holds: served a lane per element."""
+    n, rows = 2**26 - 3, 2**19
+    t = np.full((rows, 16), -100, np.int8)
+    row = np.eye(16, dtype=np.int8)[15]
+    ids = np.arange(n, dtype=np.int32) & np.int32(rows - 1)
+    d = C.to_device(t)
+    _, failure = C.scatter(d, C.to_device(ids), C.to_device(row).view((n, 16), (0, 1)), 0, add=add, out=d)
+    if add:
+        t[:, 15] += np.bincount(ids, minlength=rows).astype(np.int8)
+    else:
+        t[:] = row
+    assert failure is None and d.numpy().tobytes() == t.tobytes()
