@@ -443,7 +443,7 @@ int32_t run_plan(chelis_dag_program *prog, const chelis_gpu_tensor *const *input
                     t4[u].shape = sh4[u];
                     t4[u].strides = st4[u];
                 }
-                if (!flat || t4[0].shape[2] % 64 || !attention_causal_fits(&t4[0], &t4[1], &t4[2], &t4[3])) {
+                if (!flat || !attention_causal_fits(&t4[0], &t4[1], &t4[2], &t4[3])) {
                     s = set_error(CHELIS_HIP_EUNSUPPORTED,
                                   "dag: node %lld: attention operands are not [.., S, 64] views with a contiguous "
                                   "head axis", (long long)r.out);

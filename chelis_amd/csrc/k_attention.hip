@@ -68,10 +68,6 @@ __device__ inline float row_sum(float x) {
     return x + __shfl_xor(x, 32, 64);
 }
 
-// RAGGED: the sequence is no multiple of the tile. Rows and keys past its end
-// read the last one: such a key lies above every row's diagonal, so its
-// score is masked, and such a row is not stored.
-template <bool RAGGED>
 __global__ __launch_bounds__(kThreads, 2) void attention_causal_kernel(AttnArgs a) {
     __shared__ __attribute__((aligned(16))) float Ks[kT][kPitch];  // [key][d]
     __shared__ __attribute__((aligned(16))) float Vt[kD][kPitch];  // [d][key]
@@ -93,8 +89,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_causal_kernel(AttnArgs 
     float qf[16];
 #pragma unroll
     for (int h = 0; h < 4; ++h) {
-        const float4 x =
-            *reinterpret_cast<const float4 *>(Q + (RAGGED && row >= a.S ? a.S - 1 : row) * a.qs + 16 * q + 4 * h);
+        const float4 x = *reinterpret_cast<const float4 *>(Q + row * a.qs + 16 * q + 4 * h);
         qf[4 * h] = x.x;
         qf[4 * h + 1] = x.y;
         qf[4 * h + 2] = x.z;
@@ -114,20 +109,6 @@ __global__ __launch_bounds__(kThreads, 2) void attention_causal_kernel(AttnArgs 
 #define CHELIS_ATT_LOAD(kt)                                                                      \
     do {                                                                                         \
         const float *kp = kbase + (kt) * kT * a.ks, *vp = vbase + (kt) * kT * a.vs;              \
-        if constexpr (RAGGED) {                                                                  \
-            const int64_t k_ = (kt) * kT + skey, e_ = a.S - 1;                                   \
-            const int64_t k0_ = k_ < e_ ? k_ : e_, k1_ = k_ + 16 < e_ ? k_ + 16 : e_,            \
-                          k2_ = k_ + 32 < e_ ? k_ + 32 : e_, k3_ = k_ + 48 < e_ ? k_ + 48 : e_;  \
-            kr0 = *reinterpret_cast<const f32x4 *>(K + k0_ * a.ks + sd);                         \
-            kr1 = *reinterpret_cast<const f32x4 *>(K + k1_ * a.ks + sd);                         \
-            kr2 = *reinterpret_cast<const f32x4 *>(K + k2_ * a.ks + sd);                         \
-            kr3 = *reinterpret_cast<const f32x4 *>(K + k3_ * a.ks + sd);                         \
-            vr0 = *reinterpret_cast<const f32x4 *>(V + k0_ * a.vs + sd);                         \
-            vr1 = *reinterpret_cast<const f32x4 *>(V + k1_ * a.vs + sd);                         \
-            vr2 = *reinterpret_cast<const f32x4 *>(V + k2_ * a.vs + sd);                         \
-            vr3 = *reinterpret_cast<const f32x4 *>(V + k3_ * a.vs + sd);                         \
-            break;                                                                               \
-        }                                                                                        \
         kr0 = *reinterpret_cast<const f32x4 *>(kp);                                              \
         kr1 = *reinterpret_cast<const f32x4 *>(kp + kstep);                                      \
         kr2 = *reinterpret_cast<const f32x4 *>(kp + 2 * kstep);                                  \
@@ -240,7 +221,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_causal_kernel(AttnArgs 
 #pragma unroll
     for (int bd = 0; bd < 4; ++bd) {
         const float4 y = {acc_o[bd][0] * inv, acc_o[bd][1] * inv, acc_o[bd][2] * inv, acc_o[bd][3] * inv};
-        if (!RAGGED || row < a.S) *reinterpret_cast<float4 *>(O + row * a.os + 16 * bd + 4 * q) = y;
+        *reinterpret_cast<float4 *>(O + row * a.os + 16 * bd + 4 * q) = y;
     }
 }
 
@@ -288,7 +269,7 @@ bool attention_causal_fits(const chelis_gpu_tensor *q, const chelis_gpu_tensor *
                            const chelis_gpu_tensor *o) {
     if (!q || q->rank != 4 || !q->shape) return false;
     const int64_t B = q->shape[0], H = q->shape[1], S = q->shape[2];
-    return S > 0 && B * H > 0 && view4(q, B, H, S) && view4(k, B, H, S) && view4(v, B, H, S) &&
+    return S > 0 && S % kT == 0 && B * H > 0 && view4(q, B, H, S) && view4(k, B, H, S) && view4(v, B, H, S) &&
            view4(o, B, H, S);
 }
 
@@ -298,7 +279,7 @@ int32_t attention_causal(const chelis_gpu_tensor *q, const chelis_gpu_tensor *k,
         if (int32_t s = check_tensor(t, "attention")) return s;
     if (!attention_causal_fits(q, k, v, o))
         return set_error(CHELIS_HIP_EUNSUPPORTED,
-                         "attention: f32 [batch, heads, seq, 64] views, the last axis "
+                         "attention: f32 [batch, heads, seq, 64] views with seq a multiple of 64, the last axis "
                          "contiguous and 16-byte aligned rows");
     hipStream_t st = stream();
     if (!st) return set_error(CHELIS_HIP_EHIP, "no HIP device");
@@ -309,7 +290,7 @@ int32_t attention_causal(const chelis_gpu_tensor *q, const chelis_gpu_tensor *k,
     a.o = static_cast<float *>(o->data);
     a.heads = q->shape[1];
     a.S = q->shape[2];
-    a.qtiles = (a.S + kT - 1) / kT;
+    a.qtiles = a.S / kT;
     a.pairs = q->shape[0] * q->shape[1];
     a.q0 = q->strides[0], a.q1 = q->strides[1], a.qs = q->strides[2];
     a.k0 = k->strides[0], a.k1 = k->strides[1], a.ks = k->strides[2];
@@ -319,8 +300,7 @@ int32_t attention_causal(const chelis_gpu_tensor *q, const chelis_gpu_tensor *k,
     const int64_t blocks = a.pairs * a.qtiles;
     if (!grid_fits(blocks, kThreads)) return set_error(CHELIS_HIP_EUNSUPPORTED, "attention: grid too large");
     plan_rounds(a, blocks, device_cus());
-    if (a.S % kT) attention_causal_kernel<true><<<(unsigned)blocks, kThreads, 0, st>>>(a);
-    else attention_causal_kernel<false><<<(unsigned)blocks, kThreads, 0, st>>>(a);
+    attention_causal_kernel<<<(unsigned)blocks, kThreads, 0, st>>>(a);
     CHELIS_LAUNCH_CHECK();
     return CHELIS_HIP_OK;
 }
@@ -333,8 +313,5 @@ int32_t attention_causal(const chelis_gpu_tensor *q, const chelis_gpu_tensor *k,
 extern "C" int32_t chelis_hip_causal_attention(const chelis_gpu_tensor *q, const chelis_gpu_tensor *k,
                                                const chelis_gpu_tensor *v, double scale,
                                                const chelis_gpu_tensor *o) {
-    // the entry takes whole tiles; the programs take any sequence
-    if (q && q->rank == 4 && q->shape && q->shape[2] % 64 != 0)
-        return chelis::set_error(CHELIS_HIP_EUNSUPPORTED, "attention: seq must be a multiple of 64");
     return chelis::attention_causal(q, k, v, scale, o);
 }

@@ -208,10 +208,9 @@ extern "C" int32_t chelis_prog_transformer_block(const chelis_gpu_tensor *const 
     // reads each weight and bias where it sits, the three results landing
     // in one [3, B*S, D] block (measured at [4096,1024] x [1024,1024]: 255
     // us for the batch of three on 128-tiles against 3 x 90 us).
-    // attention as one fused launch where it applies (binary32; any length:
-    // [3, 200, 512] took four launches and 31 us in three of them), else
-    // scores, causal softmax and P.V
-    const bool fused = dt == CHELIS_DTYPE_F32 && (S % 64 == 0 || !exact_mode());
+    // attention as one fused launch where it applies (binary32, seq a
+    // multiple of 64), else scores, causal softmax and P.V
+    const bool fused = dt == CHELIS_DTYPE_F32 && S % 64 == 0;
     Workspace ws(st);
     const size_t o_h = ws.reserve(R * D * w), o_qkv = ws.reserve(3 * R * D * w),
                  o_s = ws.reserve(fused ? 0 : B * H * S * S * w),

@@ -260,3 +260,27 @@ def test_transformer_block_of_any_length(B, S):
     f = f * 0.5 * (1 + np.vectorize(erf)(f / np.sqrt(2.0)))
     ref = x + f @ w[14] + w[15]
     assert normwise(out.numpy(), ref) < 1e-5
+
+
+@pytest.mark.parametrize("S", [100, 200])
+def test_transformer_block_with_scores_of_minus_infinity_in_the_first_keys(S):
+    """Tokens of two kinds; every score of a later token against a key of the
+    first 70 is -inf: its softmax is over the others alone, and finite."""
+    D, first = 64, 70
+    f32 = np.float32
+    x = np.zeros((1, S, D), f32)
+    x[0, :first, 0], x[0, :first, 1] = 1, -1
+    x[0, first:, 2], x[0, first:, 3] = 1, -1
+    one, zero, none = np.ones(D, f32), np.zeros(D, f32), np.zeros((D, D), f32)
+    wk, bq, wv = none.copy(), zero.copy(), none.copy()
+    wk[0, 0], bq[0] = 1e37, -1e3  # q.k = -1e40 for a key of the first kind, 0 for one of the second
+    wv[2, 5] = 1
+    args = [x, one, zero, none, bq, wk, zero, wv, zero, np.eye(D, dtype=f32), zero, one, zero, np.zeros((D, 4 * D), f32),
+            np.zeros(4 * D, f32), np.zeros((4 * D, D), f32), zero]
+    out = C.empty((1, S, D), f32)
+    C.program("transformer_block", [C.to_device(a) for a in args], [out])
+    want = x[0, first:].astype(np.float64)
+    h = x[0, first:].astype(np.float64)
+    h = h / np.sqrt((h * h).mean(-1, keepdims=True) + 1e-5)
+    want[:, 5] += h[:, 2]  # the mean of equal values
+    assert normwise(out.numpy()[0, first:], want) < 1e-5
