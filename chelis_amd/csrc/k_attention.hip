@@ -180,14 +180,16 @@ __global__ __launch_bounds__(kThreads, 2) void attention_causal_kernel(AttnArgs 
                 s[kb][r] = x;
                 mx = fmaxf(mx, x);
             }
-        const float m_new = fmaxf(m_run, row_max(mx));  // key 0 <= row: finite
-        const float alpha = expf(m_run - m_new);
+        // while every score is -inf, 0 in place of the maximum keeps the
+        // exponentials 0 (-inf - -inf would be NaN, and stay)
+        const float m_new = fmaxf(m_run, row_max(mx)), m_ref = m_new == -INFINITY ? 0.f : m_new;
+        const float alpha = expf(m_run - m_ref);
         float sum = 0.f;
 #pragma unroll
         for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float p = expf(s[kb][r] - m_new);
+                const float p = expf(s[kb][r] - m_ref);
                 s[kb][r] = p;
                 sum += p;
             }

@@ -262,7 +262,7 @@ def test_transformer_block_of_any_length(B, S):
     assert normwise(out.numpy(), ref) < 1e-5
 
 
-@pytest.mark.parametrize("S", [100, 200])
+@pytest.mark.parametrize("S", [100, 128, 200])
 def test_transformer_block_with_scores_of_minus_infinity_in_the_first_keys(S):
     """Tokens of two kinds; every score of a later token against a key of the
     first 70 is -inf: its softmax is over the others alone, and finite."""
