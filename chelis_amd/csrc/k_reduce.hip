@@ -433,6 +433,10 @@ __global__ __launch_bounds__(256) void reduce_cols_chain_kernel(ChainDev ch, Lea
     const T *p[NIN];
 #pragma unroll
     for (int k = 0; k < NIN; ++k) p[k] = static_cast<const T *>(src.p[k]) + o * src.so[k] + j * src.si[k];
+    // the four-leaf steps of this thread's group that hold a leaf (an axis of
+    // three took all eight: 9.5 us against 5 for [500, 2, 2])
+    const int64_t left = (n - i0 + V - 1) / V;
+    const int nb = left < 0 ? 0 : left < NB ? (int)left : NB;
     Q in[NIN];
     auto load = [&](int t) {
 #pragma unroll
@@ -455,10 +459,10 @@ __global__ __launch_bounds__(256) void reduce_cols_chain_kernel(ChainDev ch, Lea
     };
     load(0);
 #pragma unroll 1
-    for (int t = 0; t < NB; ++t) {
+    for (int t = 0; t < nb; ++t) {
 #pragma unroll
         for (int k = 0; k < NIN; ++k) slots[k * 256 + tid] = in[k];
-        if (t + 1 < NB) load(t + 1);
+        if (t + 1 < nb) load(t + 1);
         T r[V];
         int64_t ri[V] = {0, 0, 0, 0};
         run_chain_vec<T, V>(ch, slots, NIN, tid, r);
@@ -471,7 +475,7 @@ __global__ __launch_bounds__(256) void reduce_cols_chain_kernel(ChainDev ch, Lea
     T v[NB];
     int64_t vi[NB] = {};
 #pragma unroll
-    for (int t = 0; t < NB; ++t) v[t] = tot[t][tid];
+    for (int t = 0; t < NB; ++t) v[t] = t < nb ? tot[t][tid] : identity<T, K>();
     ordered_tree<T, K, NB>(v, vi);
     // the groups of a column, in order, one level at a time
     T a = v[0];
@@ -678,7 +682,18 @@ int plan_passes(const ChainDev &ch, bool chain, const LeafSrc &src, int64_t oute
             jshift = 0;
             while (jshift < 6 && (int64_t(1) << jshift) < inner) ++jshift;
             const int64_t leaves = 8192 >> jshift;
-            if (!grid_fits(outer * ((cur_n + leaves - 1) / leaves) * ((inner + (1 << jshift) - 1) >> jshift), 256))
+            const int64_t wgs = outer * ((cur_n + leaves - 1) / leaves) * ((inner + (1 << jshift) - 1) >> jshift);
+            // many workgroups of fewer than 64 columns whose axis fills less
+            // than a twelfth (f64: a ninth) of their leaves: a thread per
+            // group (reduce_cols_kernel). 2 million leaves, f32, that kernel /
+            // this one, us: 2 columns, axis of 8 (of 4096 leaves) 11 / 336, 200
+            // 29 / 37, 400 29 / 20; 8 columns, 64 (of 1024) 29 / 33, 100 29 /
+            // 19; 32 columns, 8 (of 256) 11 / 22, 32 25 / 18; f64, 2 columns,
+            // 400 34 / 36, 3 columns, 200 (of 2048) 39 / 45, 4 columns, 400 34 /
+            // 20. Within eight workgroups per CU the few threads' length
+            // decides: 2000 leaves, axis of 8 8 / 5, 33 27 / 10. From 64
+            // columns on the other kernel leaves as many waves idle.
+            if ((inner < 64 && (sizeof(T) == 4 ? 12 : 9) * cur_n < leaves && wgs > 8 * (int64_t)device_cus()) || !grid_fits(wgs, 256))
                 jshift = -1;
         }
         const int64_t G = rows ? unit * S : (jshift >= 0 ? 8192 >> jshift : (cols4 ? 128 : 32));

@@ -339,3 +339,20 @@ def test_column_chain_leaves_on_the_vector_interpreter(dtype, n, inner):
     got = C.reduce("sum", [dx, dm], 1, chain=ch).numpy()
     assert np.array_equal(got, O.sum_axis(leaves, 1))
     assert np.array_equal(C.reduce("max", [dx, dm], 1, chain=ch).numpy(), leaves.max(1))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("outer,n,inner", [(3, 2, 2), (3, 5, 3), (9000, 3, 2), (2100, 8, 33), (2100, 11, 33), (70, 65, 3),
+                                           (2049, 85, 8), (2049, 86, 8)])
+def test_column_chain_leaves_over_short_axes(dtype, outer, n, inner):
+    """Axes that fill a small part of a workgroup's leaves, in few and in
+    many workgroups (either side of the rule that sends the many to a thread
+    per group), leaf counts off the four of an interpreter run: the same bits."""
+    rng = np.random.default_rng(n + inner)
+    x = rng.standard_normal((outer, n, inner)).astype(dtype)
+    mean = rng.standard_normal((outer, inner)).astype(dtype)
+    dx, dm = C.to_device(x), C.to_device(mean).view((outer, n, inner), (inner, 0, 1))
+    ch = C.fused_chain([("sub", 0, 1), ("mul", ("s", 0), ("s", 0))])
+    leaves = (x - mean[:, None, :]) * (x - mean[:, None, :])
+    assert np.array_equal(C.reduce("sum", [dx, dm], 1, chain=ch).numpy(), O.sum_axis(leaves, 1))
+    assert np.array_equal(C.reduce("max", [dx, dm], 1, chain=ch).numpy(), leaves.max(1))
