@@ -75,7 +75,14 @@ struct Stage16 {
     uint2 q[LAY == 1 ? 8 : 1];
 
     // element (row, k) at base[row * s_row + k * s_k]; CHECK = false: the
-    // whole tile is inside the operand and the vectors are aligned.
+    // whole tile is inside the operand. With CHECK a vector that would run
+    // past the operand is moved back to end with it, and store() puts its
+    // elements where they belong: no branch around a load, which made the
+    // compiler wait for each before the next. Rows past the operand's hold
+    // others of its values (nothing of theirs is stored); k past K is zero.
+    // LAY 0 needs K >= 8, LAY 1 four rows. (Bounds branches: 1100 x 1100 x 33
+    // bf16 13.9 us with both operands along the outer axis, 8191 x 65 x 4097
+    // 315; element by element 10.5 and 171.)
     template <bool CHECK>
     __device__ void load(const uint16_t *__restrict__ base, int64_t s_row, int64_t s_k, int64_t row0, int64_t rows,
                          int64_t k0, int64_t K) {
@@ -83,19 +90,11 @@ struct Stage16 {
         if constexpr (LAY == 1) {
             if (ACTIVE < THREADS && t >= ACTIVE) return;
             const int nb = t % 4 + 4 * (t / 32), kb = (t / 4) % 8;
-            const int64_t gr = row0 + 4 * nb;
+            const int64_t gr = row0 + 4 * nb, at = CHECK && gr + 4 > rows ? rows - 4 : gr;
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
                 const int64_t gk = k0 + 8 * kb + u;
-                const uint16_t *p = base + gr + gk * s_k;
-                if (!CHECK || (gk < K && gr + 4 <= rows)) {
-                    q[u] = load4(p);
-                } else {
-                    uint16_t e[4];
-#pragma unroll
-                    for (int w = 0; w < 4; ++w) e[w] = (gk < K && gr + w < rows) ? p[w * s_row] : (uint16_t)0;
-                    q[u] = __builtin_bit_cast(uint2, e);
-                }
+                q[u] = load4(base + at + (CHECK && gk >= K ? K - 1 : gk) * s_k);
             }
             return;
         }
@@ -104,10 +103,10 @@ struct Stage16 {
             const int idx = t + THREADS * j;
             const int row = idx / (BK / 8), kv = (idx % (BK / 8)) * 8;
             const int64_t gr = row0 + row, gk = k0 + kv;
-            const uint16_t *p = base + gr * s_row + gk * s_k;
-            if (LAY == 0 && (!CHECK || (gr < rows && gk + 8 <= K))) {
-                r[j] = load8(p);
+            if constexpr (LAY == 0) {
+                r[j] = load8(base + (CHECK && gr >= rows ? rows - 1 : gr) * s_row + (CHECK && gk + 8 > K ? K - 8 : gk));
             } else {
+                const uint16_t *p = base + gr * s_row + gk * s_k;
                 uint16_t e[8];
 #pragma unroll
                 for (int u = 0; u < 8; ++u) e[u] = (gr < rows && gk + u < K) ? p[u * s_k] : (uint16_t)0;
@@ -116,11 +115,25 @@ struct Stage16 {
         }
     }
 
-    __device__ void store(uint16_t *lds) const {
+    // row0 .. K: as the load's
+    template <bool CHECK>
+    __device__ void store(uint16_t *lds, int64_t row0, int64_t rows, int64_t k0, int64_t K) {
         const int t = threadIdx.x;
         if constexpr (LAY == 1) {
             if (ACTIVE < THREADS && t >= ACTIVE) return;
             const int nb = t % 4 + 4 * (t / 32), kb = (t / 4) % 8;
+            if (CHECK && row0 + ROWS > rows) {
+                const int64_t d = row0 + 4 * nb - (rows - 4);  // rows moved back; four and more: none of them is stored
+                const int sh = d > 0 && d < 4 ? 16 * (int)d : 0;
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    q[u] = __builtin_bit_cast(uint2, __builtin_bit_cast(uint64_t, q[u]) >> sh);
+            }
+            if (CHECK && k0 + BK > K) {
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (k0 + 8 * kb + u >= K) q[u] = uint2{0, 0};
+            }
             // output row e, word w: k = 2w in the low half, 2w + 1 in the high
             uint32_t w[4][4];
 #pragma unroll
@@ -140,6 +153,16 @@ struct Stage16 {
         for (int j = 0; j < NV; ++j) {
             const int idx = t + THREADS * j;
             const int row = idx / (BK / 8), kv = (idx % (BK / 8)) * 8;
+            if (LAY == 0 && CHECK && k0 + BK > K) {
+                const int64_t d = k0 + kv + 8 - K;  // elements moved back
+                const uint64_t lo = (uint64_t)r[j].y << 32 | r[j].x, hi = (uint64_t)r[j].w << 32 | r[j].z;
+                if (d > 0) {
+                    const int sh = 16 * (int)(d & 3);
+                    const uint64_t x = d < 4 ? lo : d < 8 ? hi : 0, y = d < 4 ? hi : 0;
+                    const uint64_t l = sh ? x >> sh | y << (64 - sh) : x, h = y >> sh;
+                    r[j] = uint4{(uint32_t)l, (uint32_t)(l >> 32), (uint32_t)h, (uint32_t)(h >> 32)};
+                }
+            }
             *reinterpret_cast<uint4 *>(lds + row * LD + kv) = r[j];
         }
     }
@@ -233,8 +256,8 @@ __global__ __launch_bounds__(THREADS) void gemm16_kernel(GemmProblem p, int64_t 
         const int64_t last = ksteps - 1;
         sa.template load<CK>(A, p.sam, p.sak, m0, p.M, 0, K);
         sb.template load<CK>(B, p.sbn, p.sbk, n0, p.N, 0, K);
-        sa.store(As[0]);
-        sb.store(Bs[0]);
+        sa.template store<CK>(As[0], m0, p.M, 0, K);
+        sb.template store<CK>(Bs[0], n0, p.N, 0, K);
         __syncthreads();
         for (int64_t ks = 0; ks < ksteps; ++ks) {
             const int buf = (int)(ks & 1);
@@ -256,8 +279,8 @@ __global__ __launch_bounds__(THREADS) void gemm16_kernel(GemmProblem p, int64_t 
 #pragma unroll
                     for (int j = 0; j < NB; ++j) acc[i][j] = mfma16<KIND>(af[i], bf[j], acc[i][j]);
             }
-            sa.store(As[buf ^ 1]);
-            sb.store(Bs[buf ^ 1]);
+            sa.template store<CK>(As[buf ^ 1], m0, p.M, kn, K);
+            sb.template store<CK>(Bs[buf ^ 1], n0, p.N, kn, K);
             __syncthreads();
         }
     };
@@ -426,12 +449,14 @@ __global__ __launch_bounds__(THREADS, 2) void gemm16_deep_kernel(GemmProblem p, 
 }
 
 // Staging layout of an operand: vectors along K (0) or along its outer
-// axis (1) where that axis has unit stride, else element by element (2);
-// *aligned: every vector starts on 16 bytes (the deep kernel's).
-int lay_of(const void *base, int64_t s_outer, int64_t s_k, int64_t s0, int64_t s1, bool *aligned) {
+// axis (1) where that axis has unit stride and holds a vector, else element
+// by element (2); *aligned: every vector starts on 16 bytes (the deep
+// kernel's).
+int lay_of(const void *base, int64_t s_outer, int64_t s_k, int64_t s0, int64_t s1, int64_t outer, int64_t K,
+           bool *aligned) {
     const bool al = (reinterpret_cast<uintptr_t>(base) & 15u) == 0 && s0 % 8 == 0 && s1 % 8 == 0;
     *aligned = al && (s_k == 1 ? s_outer : s_k) % 8 == 0;
-    return s_k == 1 ? 0 : s_outer == 1 ? 1 : 2;
+    return s_k == 1 && K >= 8 ? 0 : s_outer == 1 && outer >= 4 && K > 0 ? 1 : 2;
 }
 
 template <Narrow KIND, int ALAY, int BLAY>
@@ -447,7 +472,8 @@ int32_t gemm16_kind(const GemmProblem &p, hipStream_t st) {
     if (!grid_fits(tm * tn, 256) || nz > 65535) return set_error(CHELIS_HIP_EUNSUPPORTED, "matmul: grid too large");
     const dim3 grid((unsigned)(tm * tn), (unsigned)nz);
     bool aa, ab;
-    const int la = lay_of(p.a, p.sam, p.sak, p.sa0, p.sa1, &aa), lb = lay_of(p.b, p.sbn, p.sbk, p.sb0, p.sb1, &ab);
+    const int la = lay_of(p.a, p.sam, p.sak, p.sa0, p.sa1, p.M, p.K, &aa),
+              lb = lay_of(p.b, p.sbn, p.sbk, p.sb0, p.sb1, p.N, p.K, &ab);
     // whole tiles and whole steps with A along K: the deep kernel
     const bool whole = p.M % BM == 0 && p.N % BN == 0 && p.K % BK == 0 && p.K > 0 && aa && ab;
     if (whole && la == 0 && lb == 0) {
@@ -461,7 +487,7 @@ int32_t gemm16_kind(const GemmProblem &p, hipStream_t st) {
         return CHELIS_HIP_OK;
     }
     // instantiated layouts: both K-contiguous, A K-contiguous with B along N
-    // (row-major operands), and the element-by-element fallback
+    // (row-major operands), A along M, and the element-by-element fallback
     if (la == 0 && lb == 0) launch16<KIND, 0, 0>(p, grid, tm, tn, st);
     else if (la == 0 && lb == 1) launch16<KIND, 0, 1>(p, grid, tm, tn, st);
     else if (la == 1 && lb == 0) launch16<KIND, 1, 0>(p, grid, tm, tn, st);

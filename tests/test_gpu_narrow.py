@@ -220,3 +220,26 @@ def test_narrow_head_products_of_any_length(kind, S, D):
             ref, bound = _mm_bound(kind, np.ascontiguousarray(w[b, h]), at(v, b, h))
             got = O.narrow_decode(kind, np.ascontiguousarray(bits_of(o.numpy())[b, h])).astype(np.float64)
             assert np.all(np.abs(got - ref) <= bound)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("M,N,K", [(3, 130, 33), (4, 65, 7), (5, 131, 8), (130, 3, 9), (129, 66, 63), (131, 133, 65),
+                                   (127, 70, 71), (190, 200, 129), (258, 64, 127)])
+def test_narrow_products_at_the_vector_edges(kind, M, N, K):
+    """Operands of any odd length with either axis contiguous, one element in
+    from the allocation: a vector at the end of a row, a column or K moved
+    back to end with the operand, K shorter than a vector, fewer rows than
+    one, the guard values beside the operand never met: within the bound."""
+    a, b = finite_bits(kind, (M, K), 50 + M), finite_bits(kind, (K, N), 51 + N)
+    ref, bound = _mm_bound(kind, a, b)
+    nan = np.array([0x7FC0 if kind == "bf16" else 0x7E00] * 8, np.uint16)
+
+    def held(x, along_rows):
+        flat = np.ascontiguousarray(x.T if along_rows else x).ravel()
+        d = C.to_device(carrier(kind, np.concatenate([nan[:1], flat, nan])))
+        return d.view(x.shape, (1, x.shape[0]) if along_rows else (x.shape[1], 1), 1)
+
+    for ta in (False, True):
+        for tb in (False, True):
+            got = O.narrow_decode(kind, bits_of(C.matmul(held(a, ta), held(b, tb)).numpy())).astype(np.float64)
+            assert np.all(np.abs(got - ref) <= bound), (ta, tb)
