@@ -753,7 +753,7 @@ int32_t launch_flat(const ChainDev &ch, FlatGroups &fg, hipStream_t strm) {
 // The broadcast form: true when it takes the operands (see fused_rows_kernel)
 // and was launched; the general interpreter serves the rest (an operand
 // strided along the last axis, chains whose slots exceed 64 KiB of LDS, rows
-// shorter than a vector). The last step always runs per row: a chain of the
+// shorter than a vector, long chains over few elements). The last step always runs per row: a chain of the
 // columns alone would leave nothing in r.
 template <typename T>
 bool launch_rows_map(const ChainDev &ch, const Operands &ops, const Shape &sh, T *out, hipStream_t strm) {
@@ -779,6 +779,11 @@ bool launch_rows_map(const ChainDev &ch, const Operands &ops, const Shape &sh, T
         if (ch.op[s] == CHELIS_FUSED_CONST || (of_column(ch.a0[s]) && (one || of_column(ch.a1[s]))))
             m.step_column |= 1u << s;
     }
+    // less than a wave of vectors per SIMD: chains of more than three steps
+    // take one element per thread, a quarter (half) of the dependent work
+    // (five steps, one an exp, [1000, 33] f32 5.4 us against 7.0, [10000, 33]
+    // 7.2 / 7.1; one step 4.7 / 4.4, three 5.3 / 5.3)
+    if (ch.n_steps > 3 && m.rows * m.nv < int64_t(256) * device_cus()) return false;
     // several rows per thread only where that saves loads or steps and the
     // chip stays full: 8 waves per SIMD of 256 CUs and more
     m.R = 1;
