@@ -238,10 +238,11 @@ __global__ __launch_bounds__(THREADS, kMinWavesPerEu<T>) void gemm_mfma_kernel(G
     const int64_t in_group = bid % (GM * tiles_n);
     // this workgroup's rows and columns of C start at (mo, no); a last tile
     // that would run past the end of an operand is moved back to end with it
-    // (m0, n0), so its loads are the interior tiles' and only the elements of
-    // its own it stores. Bounds checks on every load made such tiles the
-    // stragglers of the launch: 1000 x 3000 x 4000 with both operands stored
-    // along the outer axis, 338 -> 266 us.
+    // (m0, n0) and stores only the elements of its own, so its loads are the
+    // interior tiles' where it still starts on a whole vector and K is whole
+    // steps (elsewhere each load is checked, as ever). Bounds checks on every
+    // load made such tiles the stragglers of the launch: 1000 x 3000 x 4000
+    // with both operands stored along the outer axis, 338 -> 266 us.
     const int64_t mo = (first + in_group % gsz) * BM, no = (in_group / gsz) * BN;
     const int64_t m0 = p.M >= BM && mo + BM > p.M ? p.M - BM : mo, n0 = p.N >= BN && no + BN > p.N ? p.N - BN : no;
     // causal 1: a tile wholly above the diagonal is never read (the whole

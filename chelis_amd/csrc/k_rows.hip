@@ -634,8 +634,8 @@ __device__ inline void softmax_row(T (&v)[S][V], const T *xr, T *yr, int64_t row
 
 // softmax over the last axis, optionally of where(j <= i, x * scale, -inf)
 // (causal != 0, q_len = rows per score matrix). DENSE instances serve the
-// common case (no mask, row length equal to the register capacity S*64W*V,
-// 16-byte aligned rows) with every bound test folded away. FAITHFUL as for
+// common case (no mask, row length equal to the register capacity S*L*W*V)
+// with every bound test folded away. FAITHFUL as for
 // softmax_row.
 template <typename T, int V, int S, int W, int R, int L, bool DENSE, bool RAGGED, bool FAITHFUL = false>
 __global__ __launch_bounds__(64 * W * R, W == 16 && S == 8 && (sizeof(T) == 4 || FAITHFUL) ? 8 : 1) void softmax_kernel(const T *x, T *y,
