@@ -433,10 +433,11 @@ __global__ __launch_bounds__(256) void reduce_cols_chain_kernel(ChainDev ch, Lea
     const T *p[NIN];
 #pragma unroll
     for (int k = 0; k < NIN; ++k) p[k] = static_cast<const T *>(src.p[k]) + o * src.so[k] + j * src.si[k];
-    // the four-leaf steps of this thread's group that hold a leaf (an axis of
-    // three took all eight: 9.5 us against 5 for [500, 2, 2])
+    // the four-leaf steps in which a group of this wave has a leaf, the first
+    // lane's the most (an axis of three took all eight: 9.5 us against 5 for
+    // [500, 2, 2]); one count per wave, so the loop's branch stays scalar
     const int64_t left = (n - i0 + V - 1) / V;
-    const int nb = left < 0 ? 0 : left < NB ? (int)left : NB;
+    const int nb = __builtin_amdgcn_readfirstlane(left < 0 ? 0 : left < NB ? (int)left : NB);
     Q in[NIN];
     auto load = [&](int t) {
 #pragma unroll
