@@ -351,8 +351,9 @@ def bench_bandwidth(C, H, steps, warmup):
 # the relu's known bytes fix.
 CAUSAL_READ = 8 * 16 * (512 * 513 // 2) * 4  # causal score rows read only j <= i
 BW_SET = [
-    ("softmax_f32_16384x1024", r"softmax_kernel<float,[^>]*, true, false>", 2 * 16384 * 1024 * 4),
-    ("softmax_f64_4096x4096", r"softmax_kernel<double,[^>]*, true, true>", 2 * 4096 * 4096 * 8),
+    # the softmax kernel's last arguments: dense, ragged, faithful
+    ("softmax_f32_16384x1024", r"softmax_kernel<float,[^>]*, true, false, false>", 2 * 16384 * 1024 * 4),
+    ("softmax_f64_4096x4096", r"softmax_kernel<double,[^>]*, true, false, true>", 2 * 4096 * 4096 * 8),
     ("gemv_f64_8192x8192", r"tree_wave_kernel<double", 8192 * 8192 * 8 + 2 * 8192 * 8),
     ("layer_norm_f32_65536x1024", r"layer_norm_kernel<float", 2 * 65536 * 1024 * 4),
     ("relu_f32_16384x4096", r"unary_kernel<float", 2 * 16384 * 4096 * 4),
@@ -365,7 +366,7 @@ BW_SET = [
     # the traffic is their sum
     ("reduce_sum_cols_f32_16384x4096", r"reduce_cols4_kernel<float", 16384 * 4096 * 4 + 4096 * 4, 2),
     ("softmax_adjoint_f32_65536x1024", r"softmax_adjoint_kernel<float", 3 * 65536 * 1024 * 4),
-    ("causal_softmax_f32_8x16x512x512", r"softmax_kernel<float,[^>]*, false, false>",
+    ("causal_softmax_f32_8x16x512x512", r"softmax_kernel<float,[^>]*, false, false, false>",
      CAUSAL_READ + 8 * 16 * 512 * 512 * 4),
 ]
 CALIBRATION = "relu_f32_16384x4096"
@@ -383,9 +384,9 @@ TRANSFORMER_SET = [("transformer_block_f32_b8_s512_d1024", r"gemm_mfma_kernel<fl
 # full rate on this part), so 4 * SQ_INSTS_VALU / (GRBM_GUI_ACTIVE x SIMDs)
 # is the share of the SIMDs' VALU issue capacity the dispatch used.
 VALU_SET = [
-    ("softmax_f32_16384x1024", r"softmax_kernel<float,[^>]*, true, false>"),
-    ("softmax_f64_4096x4096", r"softmax_kernel<double,[^>]*, true, true>"),
-    ("softmax_f64_4096x4096_exact", r"softmax_kernel<double,[^>]*, true, false>"),
+    ("softmax_f32_16384x1024", r"softmax_kernel<float,[^>]*, true, false, false>"),
+    ("softmax_f64_4096x4096", r"softmax_kernel<double,[^>]*, true, false, true>"),
+    ("softmax_f64_4096x4096_exact", r"softmax_kernel<double,[^>]*, true, false, false>"),
     # the binary32 default GELU (Unary 5, GeluFast; one vector per thread)
     # and dropout (the resident streaming map)
     ("gelu_f32_16384x4096", r"unary_kernel<float, \(.*Unary\)5>"),
@@ -810,6 +811,7 @@ def main(argv=None) -> int:
     if not args.no_counters:
         try:
             hrec, summary = measure_counters(kernels, args.counters_dir)
+            tdetail = "no counter rows of the headline kernel"
             if hrec is not None:
                 traffic = hrec["traffic_bytes"]
                 tdetail = (f"FETCH {hrec['fetch_bytes']} B + WRITE {hrec['write_bytes']} B per launch, median of "
