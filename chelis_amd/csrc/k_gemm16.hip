@@ -172,9 +172,9 @@ struct Stage16 {
 // 16-byte runs of a row where the layout allows. Straight from the
 // accumulators a wave's store is 32-byte pieces of four rows. (With the
 // 64-column tiles: scores and values of 8 x 16 heads of 512 x 64 bf16 61.6 ->
-// 55.4 us, of 4 heads of 64 x 64 18.4 -> 10.9, 56 heads of 777 x 64 f16 165 ->
-// 142. The deep kernel, whose tiles are whole, keeps its direct stores: staged
-// they took 2 x 8 heads of 640 x 128 from 24.8 to 26.7.)
+// 55.4 us, of 4 heads of 64 x 64 18.4 -> 10.9. The deep kernel, whose tiles
+// are whole, keeps its direct stores: staged they took 2 x 8 heads of 640 x
+// 128 from 24.8 to 26.7.)
 template <Narrow KIND, int NB>
 __device__ inline void store_tile16(const f32x4 (&acc)[4][NB], uint16_t *tile, uint16_t *C, const GemmProblem &p,
                                     int64_t m0, int64_t n0) {
